@@ -53,9 +53,9 @@ HBM_PEAK_GBS = 8000.0
 # KO 1008 + 96, equations 3952, eta 10) + 96 for the stage update
 VALU_PEAK_TFLOPS = {"fp64": 78.6, "mixed": 157.3}
 FLOP_PER_POINT_STAGE = 6788 + 96
-KERNEL_NAMES = {"fused_wide": "k_fused<interior, 256 threads, 7x7x5 tiles>",
-                "fused_thin": "k_fused<interior, 128 threads, 7x7x2 tiles>",
-                "fused_face": "k_fused<flagged faces, 256 threads>",
+KERNEL_NAMES = {"fused_wide": "k_stream<interior, 7x7x5 tiles, or that part of 7x7x7 ones>",
+                "fused_thin": "k_stream<interior, the remainder of 7x7x7 tiles>",
+                "fused_face": "k_stream<flagged faces, 256 threads> (mixed: k_fused)",
                 "fused_full": "k_fused<interior, 384 threads, 7x7x7 tiles, FP32>",
                 "derivs": "k_derivs", "rhs": "k_rhs", "face": "k_face"}
 
@@ -142,7 +142,7 @@ class Workload:
 KERNEL_SOURCES = ("dendro-gr_amd/csrc/dgr_bssn.hip", "dendro-gr_amd/csrc/stencils.h",
                   "dendro-gr_amd/csrc/bssn_rhs_phased.h", "dendro-gr_amd/csrc/bssn_rhs_generated.h",
                   "dendro-gr_amd/csrc/bssn_ham_generated.h", "dendro-gr_amd/csrc/bssn_cons_phased.h",
-                  "dendro-gr_amd/csrc/bssn_rhs_phased_gauge.h", "dendro-gr_amd/csrc/bssn_rhs_gauge_generated.h",
+                  "dendro-gr_amd/csrc/bssn_rhs_stream.h", "dendro-gr_amd/csrc/stream_fp64.h", "dendro-gr_amd/csrc/bssn_rhs_gauge_generated.h",
                   "dendro-gr_amd/build.py")
 
 

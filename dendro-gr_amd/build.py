@@ -36,19 +36,21 @@ def regenerate(verbose=False):
           os.path.join(HERE, "csrc", "bssn_rhs_generated.h")], verbose)
 
 
-# The FP64 kernels (and the rest of the library) are scheduled with the
-# iterative ILP strategy; the FP32 fused kernels, compiled from the same
-# source with DGR_F32_KERNELS in a unit of their own, keep the default one.
-MAIN_FLAGS = ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"]
+# The library's three units, compiled from one source (they differ in what they
+# instantiate and in the instruction scheduling that measured faster): host
+# code with the diagnostics' kernels, the FP32 fused kernels, the FP64 stage kernels.
+UNITS = {"main": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
+         "f32": ["-DDGR_F32_KERNELS"],
+         "stream": ["-DDGR_STREAM_KERNELS"]}
 
 
 def build_bssn(src: str, out: str, verbose: bool = False, extra=()) -> None:
-    """libdgr_bssn.so from the HIP source `src` (two units) and the C++ shim."""
+    """libdgr_bssn.so from the HIP source `src` (its units) and the C++ shim."""
     inc = ["-I", os.path.join(ROOT, "include"), "-I", os.path.join(HERE, "csrc")]
-    objs = [out + ".main.o", out + ".f32.o"]
-    # the two units compile in parallel
-    cmds = [[HIPCC, *HIP_FLAGS, *MAIN_FLAGS, *extra, "-c", *inc, src, "-o", objs[0]],
-            [HIPCC, *HIP_FLAGS, *extra, "-DDGR_F32_KERNELS", "-c", *inc, src, "-o", objs[1]]]
+    objs = [f"{out}.{u}.o" for u in UNITS]
+    # the units compile in parallel
+    cmds = [[HIPCC, *HIP_FLAGS, *flags, *extra, "-c", *inc, src, "-o", o]
+            for flags, o in zip(UNITS.values(), objs)]
     procs = []
     for c in cmds:
         if verbose:

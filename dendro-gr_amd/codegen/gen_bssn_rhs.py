@@ -15,10 +15,10 @@ The emitted function reads inputs through an accessor object
 and hands each right-hand side to `out.template put<V>(value)`, so a kernel
 decides where inputs come from and what happens to each output.
 
-Usage: python gen_bssn_rhs.py [--cse=local|global] [--phased | --ham | --cons-phased [--search]] [--gauge]
+Usage: python gen_bssn_rhs.py [--cse=local|global] [--phased | --ham | --cons-phased [--search] | --gauge]
        [output.h]
 (--phased: the right-hand side in the phase order of the fused kernel;
- --gauge: with or without --phased, the right-hand side with the gauge variants
+ --gauge: the right-hand side with the gauge variants
  of the reference's other builds, the Rochester gauge and the slow-start lapse;
  --ham: the constraints (Hamiltonian, momentum, psi4);
  --cons-phased: the constraints in the phase order of the fused constraint
@@ -649,9 +649,9 @@ def schedule_phased(defs, outs, order_vars):
     return prog
 
 
-def generate_phased(path, gauge=False):
+def generate_phased(path):
     t0 = time.time()
-    defs, outs_r, ops_after = eliminate(OUTPUTS_GAUGE if gauge else None)
+    defs, outs_r, ops_after = eliminate()
     prog = schedule_phased(defs, outs_r, PHASE_ORDER)
     vidx = [VIDX[v] for v in PHASE_ORDER]
 
@@ -680,15 +680,13 @@ def generate_phased(path, gauge=False):
             live.add(x)
         max_live = max(max_live, len(live))
         live = {y for y in live if last_use.get(y, -1) > k}
-    fn, extra = ("bssn_rhs_phased_gauge", "const T *xi, const int rochester, const T &sslt, ") if gauge \
-        else ("bssn_rhs_phased", "")
-    consts = "" if gauge else f"""
+    consts = f"""
 // first variable of the phase order (the kernel fetches it before calling)
 constexpr int kBssnFirstPhaseVar = {vidx[0]};
 // the whole phase order (variable of phase K)
 constexpr int kBssnPhaseVar[{len(vidx)}] = {{{', '.join(str(v) for v in vidx)}}};
 """
-    hdr = HEADER_TOP + (GAUGE_DOC + "// sslt is read by reference, like eta.\n" if gauge else "") + f"""//
+    hdr = HEADER_TOP + f"""//
 // Phased form for a kernel that streams the variables through LDS one at a
 // time, in the order {', '.join(PHASE_ORDER)}.
 // ctx.phase<V, NEXT, K>() (K: position of V in the order) makes variable V's
@@ -718,7 +716,7 @@ constexpr int kBssnPhaseVar[{len(vidx)}] = {{{', '.join(str(v) for v in vidx)}}}
 namespace dgr {{
 {consts}
 template <typename T, typename Ctx, typename Out>
-DGR_HD DGR_INLINE void {fn}(Ctx &ctx, const T &eta, const T *lam, const T *lamf, {extra}Out &out) {{
+DGR_HD DGR_INLINE void bssn_rhs_phased(Ctx &ctx, const T &eta, const T *lam, const T *lamf, Out &out) {{
 {chr(10).join(lines)}
 }}
 
@@ -897,7 +895,7 @@ if __name__ == "__main__":
             CSE_MODE = a.split("=", 1)[1]
     gauge = "--gauge" in sys.argv
     if "--phased" in sys.argv:
-        generate_phased(args[0] if args else "bssn_rhs_phased.h", gauge)
+        generate_phased(args[0] if args else "bssn_rhs_phased.h")
     elif "--cons-phased" in sys.argv:
         generate_cons_phased(args[0] if args else "bssn_cons_phased.h", search="--search" in sys.argv)
     elif "--ham" in sys.argv:

@@ -46,9 +46,9 @@ __host__ __device__ inline T dgr_sqrt(T x) {
 #include "stencils.h"
 #include "bssn_rhs_phased.h"
 #include "bssn_rhs_gauge_generated.h"
-#include "bssn_rhs_phased_gauge.h"
 #include "bssn_cons_phased.h"
 #include "bssn_ham_generated.h"
+#include "bssn_rhs_stream.h"
 
 namespace {
 
@@ -76,10 +76,12 @@ struct DBlock {  // device copy of a block with its grid spacing
 
 struct Tile {
     int block;
-    int q0;       // first workspace point of the tile within its chunk (split path)
+    int q0;       // first point of the tile: of its chunk's workspace (split path), of its
+                  // block's part of the RK interior buffers (fused path)
     int o[3];     // absolute index of the tile's first point along each axis
     int e[3];     // tile extents
     int lanetab;  // fused path: offset of the tile shape's lane -> point table
+    int stagetab, stagetab_halo;  // FP64 stage kernels: offsets of its staging tables
 };
 
 struct Chunk {
@@ -266,20 +268,34 @@ struct RKArgs {
     int *err;
 };
 
-// enforce_bssn_constraints on one point's values: bssn_constraints.h:15-172.
-// Order in v14: alpha, chi, gt00..gt22, At00..At22. Returns error bits.
-__device__ int enforce_point(double v14[14], double chi_floor) {
+// enforce_bssn_constraints on one point's 24 values (bssn_constraints.h:15-172),
+// in two parts so that the stage kernel can finish the metric before the
+// curvature. enforce_metric: det(gt) = 1, chi and alpha floored; returns error
+// bits, 1 (det < 0) leaving every value as it is and forbidding enforce_trace.
+__device__ __forceinline__ int enforce_metric(double *v, double chi_floor) {
 #pragma clang fp contract(off)
     const double one_third = 1.0 / 3.0;
-    double g00 = v14[2], g01 = v14[3], g02 = v14[4], g11 = v14[5], g12 = v14[6], g22 = v14[7];
-    double A00 = v14[8], A01 = v14[9], A02 = v14[10], A11 = v14[11], A12 = v14[12], A22 = v14[13];
-    int err = 0;
+    double g00 = v[12], g01 = v[13], g02 = v[14], g11 = v[15], g12 = v[16], g22 = v[17];
     double det = g00 * (g11 * g22 - g12 * g12) - g01 * g01 * g22 + 2.0 * g01 * g02 * g12 - g02 * g02 * g11;
     if (det < 0.0) return 1;
     const double s = 1.0 / pow(det, one_third);
     g00 *= s; g01 *= s; g02 *= s; g11 *= s; g12 *= s; g22 *= s;
     det = g00 * (g11 * g22 - g12 * g12) - g01 * g01 * g22 + 2.0 * g01 * g02 * g12 - g02 * g02 * g11;
-    if (fabs(det - 1.0) > 1.0e-6) err |= 2;
+    v[12] = g00; v[13] = g01; v[14] = g02; v[15] = g11; v[16] = g12; v[17] = g22;
+    if (v[1] < chi_floor) v[1] = chi_floor;
+    // std::max(alpha, CHI_FLOOR) (bssn_constraints.h:171): a NaN stays a NaN
+    // (fmax would replace it with the floor and hide it from the NaN check)
+    if (v[0] < chi_floor) v[0] = chi_floor;
+    return fabs(det - 1.0) > 1.0e-6 ? 2 : 0;
+}
+
+// tr(At) = 0 with the metric enforce_metric left
+__device__ __forceinline__ int enforce_trace(double *v) {
+#pragma clang fp contract(off)
+    const double one_third = 1.0 / 3.0;
+    const double g00 = v[12], g01 = v[13], g02 = v[14], g11 = v[15], g12 = v[16], g22 = v[17];
+    double A00 = v[18], A01 = v[19], A02 = v[20], A11 = v[21], A12 = v[22], A22 = v[23];
+    const double det = g00 * (g11 * g22 - g12 * g12) - g01 * g01 * g22 + 2.0 * g01 * g02 * g12 - g02 * g02 * g11;
     const double idet = 1.0 / det;
     const double u00 = idet * (g11 * g22 - g12 * g12);
     const double u01 = idet * (-g01 * g22 + g02 * g12);
@@ -291,14 +307,25 @@ __device__ int enforce_point(double v14[14], double chi_floor) {
     A00 -= tr3 * g00; A01 -= tr3 * g01; A02 -= tr3 * g02;
     A11 -= tr3 * g11; A12 -= tr3 * g12; A22 -= tr3 * g22;
     const double trA = A00 * u00 + A11 * u11 + A22 * u22 + 2.0 * (A01 * u01 + A02 * u02 + A12 * u12);
-    if (fabs(trA) > 1.0e-6) err |= 4;
-    v14[2] = g00; v14[3] = g01; v14[4] = g02; v14[5] = g11; v14[6] = g12; v14[7] = g22;
-    v14[8] = A00; v14[9] = A01; v14[10] = A02; v14[11] = A11; v14[12] = A12; v14[13] = A22;
-    if (v14[1] < chi_floor) v14[1] = chi_floor;
-    // std::max(alpha, CHI_FLOOR) (bssn_constraints.h:171): a NaN stays a NaN
-    // (fmax would replace it with the floor and hide it from the NaN check)
-    if (v14[0] < chi_floor) v14[0] = chi_floor;
-    return err;
+    v[18] = A00; v[19] = A01; v[20] = A02; v[21] = A11; v[22] = A12; v[23] = A22;
+    return fabs(trA) > 1.0e-6 ? 4 : 0;
+}
+
+// Both, on the 14 values they touch (alpha, chi, gt00..gt22, At00..At22).
+__device__ int enforce_point(double v14[14], double chi_floor) {
+    double v[NV];
+    v[0] = v14[0];
+    v[1] = v14[1];
+#pragma unroll
+    for (int k = 0; k < 12; k++) v[12 + k] = v14[2 + k];
+    int e = enforce_metric(v, chi_floor);
+    if (e & 1) return e;
+    e |= enforce_trace(v);
+    v14[0] = v[0];
+    v14[1] = v[1];
+#pragma unroll
+    for (int k = 0; k < 12; k++) v14[2 + k] = v[12 + k];
+    return e;
 }
 
 __device__ __forceinline__ int slot14(int v) { return v <= 1 ? v : (v >= 12 ? v - 10 : -1); }
@@ -656,20 +683,11 @@ struct StageIO {
 struct RhsPhases {
     static constexpr int N = NV;
     static constexpr bool KO = true;
-    static constexpr bool GAUGE = false;  // the standard gauge with the RIT eta(r)
     static constexpr int var(int k) { return dgr::kBssnPhaseVar[k]; }
-};
-// The right-hand side of the reference's other builds, chosen at run time:
-// BSSN_ETA_FUNCTION (eta from chi's gradient, formed in chi's phase), the
-// Rochester gauge, the slow-start lapse (its term formed in alpha's phase).
-// Its own kernels, so the default ones carry none of its registers.
-struct RhsPhasesGauge : RhsPhases {
-    static constexpr bool GAUGE = true;
 };
 struct ConsPhases {
     static constexpr int N = dgr::kConsPhases;
     static constexpr bool KO = false;
-    static constexpr bool GAUGE = false;
     static constexpr int var(int k) { return dgr::kConsPhaseVar[k]; }
 };
 
@@ -705,14 +723,7 @@ struct FusedCtx {
     double pre[PD][PREF];  // fetched region of the variables of phases K+1 .. K+PD
     double poff[PD];       // the staging offset of each fetched variable (mixed precision)
     T f[NV];               // this point's field values
-    // the eta the equations read (by reference, after the last phase): the
-    // RIT eta(r), or with P::GAUGE and eta_fn the eta of chi's gradient
-    // (BSSN_ETA_FUNCTION) set in chi's phase
-    T eta_v;
-    double eta_r0, eta_p0, eta_p1;
-    bool eta_fn, ssl_on;
-    T ssl_v;       // P::GAUGE: the slow-start lapse term (0 without it), set in alpha's phase
-    double ssl_e;  // exp(-t^2/800)
+    T eta_v;  // the RIT eta(r)
     // LDS source offsets of this thread's D_x / D_y evaluations
     int dxw[DXIT], dyw[DYIT];  // where this thread's D_x / D_y evaluations go (see dtable)
     T d1v[3], d2v[6];
@@ -922,12 +933,6 @@ struct FusedCtx {
 #pragma unroll
             for (int k = 0; k < 6; k++) DGR_PIN(d2v[k]);
         }
-        if constexpr (V == 1 && P::GAUGE) {  // chi: its first derivatives are at hand
-            if (eta_fn) eta_v = eta_function<T>(f + 12, d1v, f[1], eta_r0, eta_p0, eta_p1);
-        }
-        if constexpr (V == 0 && P::GAUGE) {
-            if (ssl_on) ssl_v = ssl_term<T>(f[0], f[1], ssl_e);
-        }
         // on a flagged face the boundary value needs the first derivatives
         if constexpr (P::KO && (m2 < 0 || FACE)) ko_term<V, S>(c, kx, ky, kz);
         if constexpr (!DEEP || m2 < 0) {
@@ -1048,6 +1053,23 @@ __device__ __forceinline__ void fused_epilogue(const StageIO &io, const T *s_ko,
         const int v = c < 2 ? c : c + 10;
         io.dst.p[v][idx] = v14[c];
     }
+}
+
+// Where the in-kernel padding refresh reads region point (gi, gj, gk) of block
+// B: a padding point inside a linked same-level neighbour at that neighbour's
+// interior point of the same coordinates (node index minus d (n - 2 PW - 1)
+// per axis), any other at its own place; the block's first point outside the
+// region. nbo: the block's 27 neighbour offsets, -1 for none.
+__device__ __forceinline__ uint64_t halo_source(const int64_t *__restrict__ nbo, const DBlock &B, bool in_region,
+                                                int gi, int gj, int gk) {
+    const int nx = B.n[0], ny = B.n[1], nz = B.n[2];
+    const int di = gi < PW ? -1 : (gi >= nx - PW ? 1 : 0);
+    const int dj = gj < PW ? -1 : (gj >= ny - PW ? 1 : 0);
+    const int dk = gk < PW ? -1 : (gk >= nz - PW ? 1 : 0);
+    const int64_t o = (in_region && (di | dj | dk)) ? nbo[(di + 1) + 3 * (dj + 1) + 9 * (dk + 1)] : -1;
+    return o >= 0 ? (uint64_t)o + (uint64_t)((gi - di * (nx - 2 * PW - 1)) +
+                                             nx * ((gj - dj * (ny - 2 * PW - 1)) + ny * (gk - dk * (nz - 2 * PW - 1))))
+                  : B.offset + (uint64_t)(in_region ? gi + nx * (gj + ny * gk) : 0);
 }
 
 // Tile geometry, this thread's point, the region elements it fetches and its
@@ -1181,22 +1203,8 @@ __device__ __forceinline__ void fused_tile(const StageIO &io, const RhsParams &p
             ctx.sig_gauge = ctx.sig_other = T(prm.ko_sigma);
         }
     }
-    // eta: the RIT eta(r), or (P::GAUGE with eta_func) set in chi's phase from
-    // chi's gradient
-    if (P::GAUGE && prm.eta_func)
-        ctx.eta_v = T(0);
-    else
-        ctx.eta_v = T(rit_eta(coord(B.pmin[0], ctx.ax, B.h[0]), coord(B.pmin[1], ctx.ay, B.h[1]),
-                              coord(B.pmin[2], ctx.az, B.h[2]), prm));
-    ctx.eta_r0 = prm.eta_r0;
-    ctx.eta_p0 = prm.eta_p0;
-    ctx.eta_p1 = prm.eta_p1;
-    if constexpr (P::GAUGE) {
-        ctx.eta_fn = prm.eta_func != 0;
-        ctx.ssl_on = prm.ssl != 0;
-        ctx.ssl_e = prm.ssl_dev ? prm.ssl_dev[1] : prm.ssl_e;
-        ctx.ssl_v = T(0);
-    }
+    ctx.eta_v = T(rit_eta(coord(B.pmin[0], ctx.ax, B.h[0]), coord(B.pmin[1], ctx.ay, B.h[1]),
+                          coord(B.pmin[2], ctx.az, B.h[2]), prm));
     const T lam[4] = {T(prm.lam[0]), T(prm.lam[1]), T(prm.lam[2]), T(prm.lam[3])};
     const T lamf[2] = {T(prm.lamf[0]), T(prm.lamf[1])};
     ctx.template fetch<0>();
@@ -1205,12 +1213,7 @@ __device__ __forceinline__ void fused_tile(const StageIO &io, const RhsParams &p
     static_assert(C::PD <= 3, "prefetch distance");
     ctx.begin();
     FusedOut<FACE, C, T, HALO, P> out(ctx);
-    if constexpr (P::GAUGE) {
-        const T xi[3] = {T(prm.xi[0]), T(prm.xi[1]), T(prm.xi[2])};
-        dgr::bssn_rhs_phased_gauge<T>(ctx, ctx.eta_v, lam, lamf, xi, prm.rochester, ctx.ssl_v, out);
-    } else {
-        dgr::bssn_rhs_phased<T>(ctx, ctx.eta_v, lam, lamf, out);
-    }
+    dgr::bssn_rhs_phased<T>(ctx, ctx.eta_v, lam, lamf, out);
     if (active) fused_epilogue<C, T>(io, s_ko, ctx.f, ctx.tid, idx, q, prm.chi_floor);
 }
 
@@ -1221,7 +1224,7 @@ __device__ __forceinline__ void fused_tile(const StageIO &io, const RhsParams &p
 #define DGR_FP32_WAVES 2  // waves per SIMD the FP32 kernels are built for
 #endif
 
-template <bool FACE, class C, typename T, bool HALO = false, bool GAUGE = false>
+template <bool FACE, class C, typename T, bool HALO = false>
 __global__ __launch_bounds__(C::FT, sizeof(T) < sizeof(double) ? DGR_FP32_WAVES : 1) void k_fused(
     const StageIO io, const RhsParams prm, const DBlock *__restrict__ blocks,
     const dgr::AxisConsts *__restrict__ bconst, const Tile *__restrict__ tiles,
@@ -1236,9 +1239,13 @@ __global__ __launch_bounds__(C::FT, sizeof(T) < sizeof(double) ? DGR_FP32_WAVES 
 
     const Tile tl = tiles[blockIdx.x];
     const DBlock B = blocks[tl.block];
-    fused_tile<FACE, C, T, HALO, std::conditional_t<GAUGE, RhsPhasesGauge, RhsPhases>>(
-        io, prm, tl, B, bconst + 3 * (size_t)tl.block, tabs, dtab, s_tile, s_dx, s_dy, s_ko);
+    fused_tile<FACE, C, T, HALO>(io, prm, tl, B, bconst + 3 * (size_t)tl.block, tabs, dtab, s_tile, s_dx, s_dy,
+                                 s_ko);
 }
+
+#ifndef DGR_F32_KERNELS
+#include "stream_fp64.h"
+#endif
 
 struct ConsPtrs {
     double *c[6];  // ham, mom0, mom1, mom2, psi4 real, psi4 imaginary (any may be null)
@@ -2022,8 +2029,29 @@ extern "C" __attribute__((visibility("hidden"))) void dgr_internal_fused_f32_ker
     k[6] = reinterpret_cast<const void *>(&k_fused<false, CfgFull, float, true>);
     k[7] = reinterpret_cast<const void *>(&k_fused<true, CfgOf<float>::Wide, float, true>);
 }
+#elif defined(DGR_STREAM_KERNELS)
+// The FP64 stage kernels (stream_fp64.h), [halo][gauge][wide, full, face]
+extern "C" __attribute__((visibility("hidden"))) void dgr_internal_stream_kernels(const void **k) {
+#ifdef DGR_PROBE
+    k[0] = reinterpret_cast<const void *>(&DGR_PROBE);
+#else
+    k[0] = reinterpret_cast<const void *>(&k_stream<false, SWide, false, false>);
+    k[1] = reinterpret_cast<const void *>(&k_stream<false, SFull, false, false>);
+    k[2] = reinterpret_cast<const void *>(&k_stream<true, SWide, false, false>);
+    k[3] = reinterpret_cast<const void *>(&k_stream<false, SWide, false, true>);
+    k[4] = reinterpret_cast<const void *>(&k_stream<false, SFull, false, true>);
+    k[5] = reinterpret_cast<const void *>(&k_stream<true, SWide, false, true>);
+    k[6] = reinterpret_cast<const void *>(&k_stream<false, SWide, true, false>);
+    k[7] = reinterpret_cast<const void *>(&k_stream<false, SFull, true, false>);
+    k[8] = reinterpret_cast<const void *>(&k_stream<true, SWide, true, false>);
+    k[9] = reinterpret_cast<const void *>(&k_stream<false, SWide, true, true>);
+    k[10] = reinterpret_cast<const void *>(&k_stream<false, SFull, true, true>);
+    k[11] = reinterpret_cast<const void *>(&k_stream<true, SWide, true, true>);
+#endif
+}
 #else
 extern "C" void dgr_internal_fused_f32_kernels(const void **k);
+extern "C" void dgr_internal_stream_kernels(const void **k);
 
 namespace {
 // Device scratch of dgr_constraint_l2_norm_noalloc: the norm's per-workgroup
@@ -2071,14 +2099,15 @@ struct dgr_plan {
     double *d_stage = nullptr;  // split path RK4: 2 * 24 * szpdof (stage state, accumulator)
     bool fused = true;          // k_fused (default) or the split k_derivs/k_rhs path (DGR_KERNEL=split)
     int precision = DGR_PRECISION_FP64;  // arithmetic of the fused kernel
-    // k_fused tiles per precision (0 FP64, 1 mixed), XCD-grouped, group k in
+    // tile lists (LIST_FP64, LIST_MIXED, LIST_CONS), XCD-grouped, group k in
     // [fgroup[p][k], fgroup[p][k+1]), each interior block tiled by the scheme
     // tiling[p] holds for its size (else the default of tiling_of)
-    Tile *d_ftiles[2] = {};
-    int fgroup[2][NFGROUP + 1] = {};
+    Tile *d_ftiles[3] = {};
+    int fgroup[3][NFGROUP + 1] = {};
     std::map<std::array<int, 3>, int> tiling[2];
     std::vector<DBlock> hblocks;                  // host copy of the block table
     std::map<std::array<int, 4>, int> lane_off;   // lane table offset per (ex, ey, ez, threads)
+    std::map<std::array<int, 3>, int> stage_off;  // staging table offset per (ex, threads, halo)
     dgr::AxisConsts *d_bconst = nullptr;  // k_fused: x, y, z stencil constants per block
     uint16_t *d_tabs = nullptr;           // k_fused: lane tables per tile shape, slot tables per config
     int dtab_wide = 0, dtab_thin = 0, dtab_full = 0;  // offsets of the configurations' slot tables
@@ -2119,7 +2148,13 @@ struct dgr_plan {
     // optional per-kernel timing: event pairs recorded around each launch
     bool timing = false;
     std::vector<hipEvent_t> event_pool;
-    std::vector<std::pair<hipEvent_t, hipEvent_t>> pending[DGR_TIMING_KINDS];
+    struct Timed {
+        hipEvent_t a, b;
+        double share;  // of the launch's time
+        bool last;     // the launch's last entry: its events go back to the pool
+    };
+    std::vector<Timed> pending[DGR_TIMING_KINDS];
+    double full_regular = 1.0;  // FP64 list: the 5-deep part's share of the points of the 6-7 deep tiles
 
     hipEvent_t take_event() {
         if (event_pool.empty()) {
@@ -2141,7 +2176,9 @@ namespace {
 // stencil tap (8-byte words: conflict-free both for 32 banks serving 16 lanes
 // and 64 banks serving 32 lanes per cycle). Points beyond ft/32 in a residue
 // class take free lanes; lanes still free repeat a point of their own residue
-// class (same address, so no conflict) and store nothing.
+// class (same address, so no conflict) and store nothing. The second half
+// numbers the lanes that hold a point of their own (a repeating lane has its
+// point's number).
 void lane_table(int ex, int ey, int ez, int ft, std::vector<uint16_t> &out) {
     const int n = ex * ey * ez, groups = ft / 32;
     std::vector<std::vector<int>> res(32);
@@ -2166,6 +2203,12 @@ void lane_table(int ex, int ey, int ez, int ft, std::vector<uint16_t> &out) {
             out.push_back((uint16_t)((rr.empty() ? 0 : rr[0]) | LANE_SHADOW));
         }
     }
+    std::vector<uint16_t> rank(n);
+    uint16_t next = 0;
+    for (int l = 0; l < ft; l++)
+        if (lane[l] >= 0) rank[lane[l]] = next++;
+    const size_t first = out.size() - ft;
+    for (int l = 0; l < ft; l++) out.push_back(rank[out[first + l] & (LANE_SHADOW - 1)]);
 }
 
 // Slot table of a tile configuration: slot (it, tid) -> the position
@@ -2207,6 +2250,48 @@ bool dtable(std::vector<uint16_t> &out) {
     return ok;
 }
 
+// Staging table of an FP64 stage kernel's configuration: (pass, thread) -> where
+// in the staged region (column + 13 row, row = j + 13 k) the pair of neighbours
+// starts that the thread reads. The order of SCfg: first the pairs every
+// variable needs. Without HALO a row's pairs start at columns 0 2 4 6 8 10 11
+// (no further than ex + 4: the region's last two columns); with HALO
+// at 0 1 | 3 5 7 8 | 10 11, the parts left of, in and right of a tile of ex = 7
+// points, so that each part can come from another block (shorter tiles
+// likewise). Idle threads repeat the last pair of the table.
+template <class C>
+bool stage_table(bool halo, int ex, std::vector<uint16_t> &out) {
+    std::vector<int> inner, outer;  // pair columns: the tile's own, and the others
+    if (halo) {
+        for (int k = 0; k < 4; k++) inner.push_back(std::min(3 + 2 * k, ex + 1));
+        outer = {0, 1, 3 + ex, 4 + ex};
+    } else {
+        for (int c : {2, 4, 6, 8}) inner.push_back(std::min(c, ex + 4));
+        for (int c : {0, 10, 11}) outer.push_back(std::min(c, ex + 4));
+    }
+    std::vector<uint16_t> slots;
+    // rows by how often they lie outside the tile along y and z
+    auto rows = [&](int outside, const std::vector<int> &cols) {
+        for (int k = 0; k < C::FZ + 2 * PW; k++)
+            for (int j = 0; j < RMAX; j++) {
+                const int o = (k < PW || k >= PW + C::FZ) + (j < PW || j >= PW + TMAX);
+                if (o != outside) continue;
+                for (int c : cols) slots.push_back((uint16_t)(c + FRX * (j + RMAX * k)));
+            }
+    };
+    std::vector<int> row(inner);
+    row.insert(row.end(), outer.begin(), outer.end());
+    std::sort(row.begin(), row.end());
+    rows(0, row);
+    rows(1, inner);
+    bool ok = (int)slots.size() == C::cross(halo);
+    rows(1, outer);
+    rows(2, inner);
+    ok = ok && (int)slots.size() == C::all(halo);
+    slots.resize((size_t)C::passes(halo) * C::FT, slots.back());
+    out.insert(out.end(), slots.begin(), slots.end());
+    return ok;
+}
+
 // m interior points -> ceil(m/emax) near-equal parts of at most emax points
 void split_axis_max(int m, int emax, std::vector<std::pair<int, int>> &parts) {
     const int np = (m + emax - 1) / emax;
@@ -2222,11 +2307,19 @@ int thread_count(int group) {
     return group == FG_THIN ? CfgThin::FT : group == FG_FULL ? CfgFull::FT : CfgWide::FT;
 }
 
-// Appends the tiles of block b under scheme `sch` to per[group][slot]. Blocks
+// The tile lists of a plan: the FP64 stage kernels', the mixed-precision ones'
+// and the constraints'.
+enum { LIST_FP64 = 0, LIST_MIXED = 1, LIST_CONS = 2, NLIST = 3 };
+
+// Appends list `p`'s tiles of block b under scheme `sch` to per[group][slot].
+// In the FP64 list a remainder of 1-2 points joins the 5 before it in a tile of
+// the 7-deep shape: a thin tile of its own stages and differentiates 6 planes
+// of halo for its 2 (on 13^3 blocks, 4096 of them, the two launches of a stage
+// fetched 3.3 GB where one fetches 2.4). Blocks
 // with flagged faces are cut along z into near-equal parts of at most 5 (each
 // >= 4 points, so the one-sided closures, which reach 5 points along their
 // axis, stay inside the staged region), whatever the scheme.
-void block_tiles(const DBlock &d, uint32_t b, int sch, std::vector<std::vector<Tile>> *per, size_t slot) {
+void block_tiles(const DBlock &d, uint32_t b, int p, int sch, std::vector<std::vector<Tile>> *per, size_t slot) {
     std::vector<std::pair<int, int>> px, py, pz;
     split_axis_max(d.n[0] - 6, TMAX, px);
     split_axis_max(d.n[1] - 6, TMAX, py);
@@ -2236,22 +2329,24 @@ void block_tiles(const DBlock &d, uint32_t b, int sch, std::vector<std::vector<T
         split_axis_max(d.n[2] - 6, CfgFull::FZ, pz);
     } else {
         for (int o = PW, m = d.n[2] - 6; m > 0;) {
-            const int e = std::min(m, CfgWide::FZ);
+            const int e = std::min(m, p == LIST_FP64 && m <= CfgFull::FZ ? CfgFull::FZ : CfgWide::FZ);
             pz.push_back({o, e});
             o += e;
             m -= e;
         }
     }
+    int q0 = 0;
     for (auto &z : pz)
         for (auto &y : py)
             for (auto &x : px) {
                 Tile t{};
                 t.block = (int)b;
-                t.q0 = 0;
+                t.q0 = q0;
+                q0 += x.second * y.second * z.second;
                 t.o[0] = x.first; t.o[1] = y.first; t.o[2] = z.first;
                 t.e[0] = x.second; t.e[1] = y.second; t.e[2] = z.second;
                 const int g = d.bflag                                    ? FG_FACE
-                              : sch == SCH_FULL                          ? FG_FULL
+                              : sch == SCH_FULL || t.e[2] > CfgWide::FZ  ? FG_FULL
                               : sch == SCH_WT && t.e[2] <= CfgThin::FZ ? FG_THIN
                                                                          : FG_WIDE;
                 per[g][slot].push_back(t);
@@ -2298,7 +2393,7 @@ int tiling_of(const dgr_plan *plan, int p, const DBlock &d) {
     return SCH_WT;
 }
 
-// Sets lanetab of every tile from the plan's lane tables (all shapes exist).
+// Sets the table offsets of every tile from the plan's tables (all shapes exist).
 bool assign_lane_tables(const dgr_plan *plan, std::vector<Tile> &tiles, const int *fgroup) {
     for (int g = 0; g < NFGROUP; g++)
         for (int i = fgroup[g]; i < fgroup[g + 1]; i++) {
@@ -2306,6 +2401,10 @@ bool assign_lane_tables(const dgr_plan *plan, std::vector<Tile> &tiles, const in
             auto it = plan->lane_off.find({t.e[0], t.e[1], t.e[2], thread_count(g)});
             if (it == plan->lane_off.end()) return false;
             t.lanetab = it->second;
+            const auto plain = plan->stage_off.find({t.e[0], thread_count(g), 0});
+            const auto halo = plan->stage_off.find({t.e[0], thread_count(g), 1});
+            t.stagetab = plain == plan->stage_off.end() ? 0 : plain->second;
+            t.stagetab_halo = halo == plan->stage_off.end() ? 0 : halo->second;
         }
     return true;
 }
@@ -2317,12 +2416,21 @@ hipError_t build_ftiles(dgr_plan *plan, int p) {
     for (auto &v : per) v.resize(nb);
     for (size_t b = 0; b < nb; b++) {
         const DBlock &d = plan->hblocks[b];
-        block_tiles(d, (uint32_t)b, d.bflag ? SCH_WT : tiling_of(plan, p, d), per, b);
+        block_tiles(d, (uint32_t)b, p, d.bflag ? SCH_WT : tiling_of(plan, p == LIST_MIXED, d), per, b);
     }
     std::vector<Tile> tiles;
     int fg[NFGROUP + 1];
     group_tiles(per, tiles, fg);
     if (!assign_lane_tables(plan, tiles, fg)) return hipErrorInvalidValue;
+    if (p == LIST_FP64) {
+        double regular = 0.0, all = 0.0;
+        for (int i = fg[FG_FULL]; i < fg[FG_FULL + 1]; i++) {
+            const int *e = tiles[i].e;
+            regular += (double)e[0] * e[1] * CfgWide::FZ;
+            all += (double)e[0] * e[1] * e[2];
+        }
+        plan->full_regular = all > 0.0 ? regular / all : 1.0;
+    }
     Tile *d = nullptr;
     hipError_t e = hipSuccess;
     if (!tiles.empty()) {
@@ -2484,6 +2592,14 @@ int dgr_plan_create(int device, const dgr_block *blocks, uint32_t nblocks, uint6
     tabs_ok = dtable<CfgThin>(tabs) && tabs_ok;
     plan->dtab_full = (int)tabs.size();
     tabs_ok = dtable<CfgFull>(tabs) && tabs_ok;
+    // (blocks are at least 13 wide, so near-equal parts are 4 to 7 points)
+    for (int ex = 4; ex <= TMAX; ex++)
+        for (int halo = 0; halo < 2; halo++) {
+            plan->stage_off[{ex, SWide::FT, halo}] = (int)tabs.size();
+            tabs_ok = stage_table<SWide>(halo, ex, tabs) && tabs_ok;
+            plan->stage_off[{ex, SFull::FT, halo}] = (int)tabs.size();
+            tabs_ok = stage_table<SFull>(halo, ex, tabs) && tabs_ok;
+        }
     if (!tabs_ok) {
         dgr_plan_destroy(plan);
         return fail(DGR_E_INVALID, "internal error: D_x / D_y slot table does not match its configuration");
@@ -2497,7 +2613,7 @@ int dgr_plan_create(int device, const dgr_block *blocks, uint32_t nblocks, uint6
             for (int sch = 0; sch < (d.bflag ? 1 : NSCHEME); sch++) {
                 std::vector<std::vector<Tile>> per[NFGROUP];
                 for (auto &v : per) v.resize(1);
-                block_tiles(d, b, sch, per, 0);
+                for (int p = 0; p < NLIST; p++) block_tiles(d, b, p, sch, per, 0);
                 for (int g = 0; g < NFGROUP; g++)
                     for (const Tile &t : per[g][0]) {
                         const std::array<int, 4> key{t.e[0], t.e[1], t.e[2], thread_count(g)};
@@ -2530,7 +2646,7 @@ int dgr_plan_create(int device, const dgr_block *blocks, uint32_t nblocks, uint6
     if (e == hipSuccess && !wg_tile.empty()) e = hipMemcpy(plan->d_wg_tile, wg_tile.data(), sizeof(int) * wg_tile.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess && !face_tiles.empty())
         e = hipMemcpy(plan->d_face_tiles, face_tiles.data(), sizeof(int) * face_tiles.size(), hipMemcpyHostToDevice);
-    for (int p = 0; p < 2 && e == hipSuccess; p++) e = build_ftiles(plan, p);
+    for (int p = 0; p < NLIST && e == hipSuccess; p++) e = build_ftiles(plan, p);
     if (e == hipSuccess) e = hipMemset(plan->d_err, 0, sizeof(int));
     if (e != hipSuccess) {
         dgr_plan_destroy(plan);
@@ -2546,8 +2662,9 @@ int dgr_plan_destroy(dgr_plan *plan) {
     (void)hipSetDevice(plan->device);
     for (auto &v : plan->pending)
         for (auto &pr : v) {
-            (void)hipEventDestroy(pr.first);
-            (void)hipEventDestroy(pr.second);
+            if (!pr.last) continue;
+            (void)hipEventDestroy(pr.a);
+            (void)hipEventDestroy(pr.b);
         }
     for (hipEvent_t e : plan->event_pool) (void)hipEventDestroy(e);
     (void)hipFree(plan->d_blocks);
@@ -2558,6 +2675,7 @@ int dgr_plan_destroy(dgr_plan *plan) {
     (void)hipFree(plan->d_stage);
     (void)hipFree(plan->d_ftiles[0]);
     (void)hipFree(plan->d_ftiles[1]);
+    (void)hipFree(plan->d_ftiles[2]);
     (void)hipFree(plan->d_bconst);
     (void)hipFree(plan->d_tabs);
     (void)hipFree(plan->d_istage);
@@ -2640,12 +2758,13 @@ int dgr_plan_kernel_times(dgr_plan *plan, double *ms, int64_t *launches) {
         ms[k] = 0.0;
         launches[k] = (int64_t)plan->pending[k].size();
         for (auto &pr : plan->pending[k]) {
-            HIP_OK(hipEventSynchronize(pr.second));
+            HIP_OK(hipEventSynchronize(pr.b));
             float t = 0.f;
-            HIP_OK(hipEventElapsedTime(&t, pr.first, pr.second));
-            ms[k] += t;
-            plan->event_pool.push_back(pr.first);
-            plan->event_pool.push_back(pr.second);
+            HIP_OK(hipEventElapsedTime(&t, pr.a, pr.b));
+            ms[k] += pr.share * t;
+            if (!pr.last) continue;
+            plan->event_pool.push_back(pr.a);
+            plan->event_pool.push_back(pr.b);
         }
         plan->pending[k].clear();
     }
@@ -2695,8 +2814,10 @@ int load_ptrs(VarPtrs &vp, const double *const *src, const char *what) {
 }
 
 // Runs `launch` on `st`, bracketed by timing events when the plan records them.
+// With `also` >= 0 (above `kind`) the launch counts there too, with the rest of
+// its time.
 template <typename F>
-void timed(dgr_plan *plan, int kind, hipStream_t st, F launch) {
+void timed(dgr_plan *plan, int kind, hipStream_t st, F launch, int also = -1, double share = 1.0) {
     if (!plan->timing) {
         launch();
         return;
@@ -2706,7 +2827,8 @@ void timed(dgr_plan *plan, int kind, hipStream_t st, F launch) {
     launch();
     const bool rb = b && hipEventRecord(b, st) == hipSuccess;
     if (ra && rb) {
-        plan->pending[kind].push_back({a, b});
+        plan->pending[kind].push_back({a, b, share, also < 0});
+        if (also >= 0) plan->pending[also].push_back({a, b, 1.0 - share, true});
     } else {  // an unrecorded pair would fail in dgr_plan_kernel_times: drop it
         if (a) plan->event_pool.push_back(a);
         if (b) plan->event_pool.push_back(b);
@@ -2747,7 +2869,12 @@ int run_chunks(dgr_plan *plan, const VarPtrs &state, const VarPtrs &rhs, const R
 template <bool FACE, class C, typename T, bool HALO, bool GAUGE = false>
 const void *fused_kernel() {
     if constexpr (sizeof(T) == sizeof(double)) {
-        return reinterpret_cast<const void *>(&k_fused<FACE, C, T, HALO, GAUGE>);
+        static const void *const *tab = [] {
+            static const void *k[12];
+            dgr_internal_stream_kernels(k);
+            return k;
+        }();
+        return tab[6 * HALO + 3 * GAUGE + (FACE ? 2 : C::FT == CfgFull::FT ? 1 : 0)];
     } else {
         static_assert(!GAUGE, "the gauge variants are FP64 only");
         static const void *const *tab = [] {
@@ -2763,56 +2890,80 @@ const void *fused_kernel() {
     }
 }
 
+StreamIO stream_io(const StageIO &io, const RhsParams &prm) {
+    StreamIO r{};
+    r.prm = prm;
+    const bool rk = io.stage >= 0;
+    r.src = io.src;
+    r.dst = rk ? io.dst : io.rhs;
+    r.u0 = rk ? io.u0.p[0] : nullptr;
+    r.acc = rk ? io.acc.p[0] : nullptr;
+    r.cacc = io.cacc;
+    r.cnext = !rk ? 1.0 : io.stage == 3 ? io.cacc : io.cnext;
+    r.stage = io.stage;
+    r.enforce = io.stage == 3 || (rk && io.enforce_stage);
+    r.err = io.err;
+    r.nbo = io.nbo;
+    return r;
+}
+
 template <bool FACE, class C, typename T, bool HALO = false, bool GAUGE = false>
 void launch_fused(dgr_plan *plan, const Tile *tiles, const int *fg, int group, int dtab, const StageIO &io,
                   const RhsParams &prm, hipStream_t st) {
     const int n = fg[group + 1] - fg[group];
     if (!n) return;
-    // k_fused's parameters, in order
-    StageIO a_io = io;
+    // the kernel's parameters, in order (StreamIO holds the RhsParams)
+    constexpr bool FP64 = sizeof(T) == sizeof(double);
+    std::conditional_t<FP64, StreamIO, StageIO> a_io;
+    if constexpr (FP64) a_io = stream_io(io, prm);
+    else a_io = io;
     RhsParams a_prm = prm;
     const DBlock *a_blocks = plan->d_blocks;
     const dgr::AxisConsts *a_bconst = plan->d_bconst;
     const Tile *a_tiles = tiles + fg[group];
     const uint16_t *a_tabs = plan->d_tabs;
     int a_dtab = dtab;
-    void *args[] = {&a_io, &a_prm, &a_blocks, &a_bconst, &a_tiles, &a_tabs, &a_dtab};
-    timed(plan, 3 + group, st, [&] {
-        (void)hipLaunchKernel(fused_kernel<FACE, C, T, HALO, GAUGE>(), dim3(n), dim3(C::FT), args, 0, st);
-    });
+    void *all[] = {&a_io, &a_prm, &a_blocks, &a_bconst, &a_tiles, &a_tabs, &a_dtab};
+    if (FP64) all[1] = all[0];
+    void **args = all + FP64;
+    // an FP64 launch on 6-7 deep tiles counts as the regular and the thin one it
+    // replaces, its time divided by their points
+    const bool merged = FP64 && group == FG_FULL;
+    timed(
+        plan, 3 + (merged ? FG_WIDE : group), st,
+        [&] { (void)hipLaunchKernel(fused_kernel<FACE, C, T, HALO, GAUGE>(), dim3(n), dim3(C::FT), args, 0, st); },
+        merged ? 3 + FG_THIN : -1, merged ? plan->full_regular : 1.0);
 }
 
-// The launches of one tile list (groups as in fg).
+// The FP64 launches of one tile list (groups as in fg).
+template <bool HALO, bool GAUGE>
+void launch_stream(dgr_plan *plan, const Tile *tiles, const int *fg, const StageIO &io, const RhsParams &prm,
+                   hipStream_t st) {
+    launch_fused<false, CfgWide, double, HALO, GAUGE>(plan, tiles, fg, FG_WIDE, plan->dtab_wide, io, prm, st);
+    launch_fused<false, CfgFull, double, HALO, GAUGE>(plan, tiles, fg, FG_FULL, plan->dtab_full, io, prm, st);
+    launch_fused<true, CfgWide, double, HALO, GAUGE>(plan, tiles, fg, FG_FACE, plan->dtab_wide, io, prm, st);
+}
+
 template <typename T>
 void launch_fused_all(dgr_plan *plan, const Tile *tiles, const int *fg, const StageIO &io, const RhsParams &prm,
                       hipStream_t st) {
     if constexpr (sizeof(T) == sizeof(double)) {
-        if (gauge_variant(prm)) {  // the reference's other builds (FP64 only)
-            if (io.nbo) {
-                launch_fused<false, CfgWide, T, true, true>(plan, tiles, fg, FG_WIDE, plan->dtab_wide, io, prm, st);
-                launch_fused<false, CfgThin, T, true, true>(plan, tiles, fg, FG_THIN, plan->dtab_thin, io, prm, st);
-                launch_fused<true, CfgWide, T, true, true>(plan, tiles, fg, FG_FACE, plan->dtab_wide, io, prm, st);
-            } else {
-                launch_fused<false, CfgWide, T, false, true>(plan, tiles, fg, FG_WIDE, plan->dtab_wide, io, prm, st);
-                launch_fused<false, CfgThin, T, false, true>(plan, tiles, fg, FG_THIN, plan->dtab_thin, io, prm, st);
-                launch_fused<true, CfgWide, T, false, true>(plan, tiles, fg, FG_FACE, plan->dtab_wide, io, prm, st);
-            }
-            return;
-        }
-    }
-    if (io.nbo) {  // the padding refresh inside the stage kernel
-        launch_fused<false, typename CfgOf<T>::Wide, T, true>(plan, tiles, fg, FG_WIDE, plan->dtab_wide, io, prm, st);
-        launch_fused<false, typename CfgOf<T>::Thin, T, true>(plan, tiles, fg, FG_THIN, plan->dtab_thin, io, prm, st);
-        if constexpr (sizeof(T) < sizeof(double))
-            launch_fused<false, CfgFull, T, true>(plan, tiles, fg, FG_FULL, plan->dtab_full, io, prm, st);
-        launch_fused<true, typename CfgOf<T>::Wide, T, true>(plan, tiles, fg, FG_FACE, plan->dtab_wide, io, prm, st);
-        return;
-    }
-    launch_fused<false, typename CfgOf<T>::Wide, T>(plan, tiles, fg, FG_WIDE, plan->dtab_wide, io, prm, st);
-    launch_fused<false, typename CfgOf<T>::Thin, T>(plan, tiles, fg, FG_THIN, plan->dtab_thin, io, prm, st);
-    if constexpr (sizeof(T) < sizeof(double))
+        const bool gauge = gauge_variant(prm);  // the reference's other builds (FP64 only)
+        if (io.nbo && gauge) launch_stream<true, true>(plan, tiles, fg, io, prm, st);
+        else if (io.nbo) launch_stream<true, false>(plan, tiles, fg, io, prm, st);
+        else if (gauge) launch_stream<false, true>(plan, tiles, fg, io, prm, st);
+        else launch_stream<false, false>(plan, tiles, fg, io, prm, st);
+    } else if (io.nbo) {  // the padding refresh inside the stage kernel
+        launch_fused<false, CfgOf<float>::Wide, T, true>(plan, tiles, fg, FG_WIDE, plan->dtab_wide, io, prm, st);
+        launch_fused<false, CfgOf<float>::Thin, T, true>(plan, tiles, fg, FG_THIN, plan->dtab_thin, io, prm, st);
+        launch_fused<false, CfgFull, T, true>(plan, tiles, fg, FG_FULL, plan->dtab_full, io, prm, st);
+        launch_fused<true, CfgOf<float>::Wide, T, true>(plan, tiles, fg, FG_FACE, plan->dtab_wide, io, prm, st);
+    } else {
+        launch_fused<false, CfgOf<float>::Wide, T>(plan, tiles, fg, FG_WIDE, plan->dtab_wide, io, prm, st);
+        launch_fused<false, CfgOf<float>::Thin, T>(plan, tiles, fg, FG_THIN, plan->dtab_thin, io, prm, st);
         launch_fused<false, CfgFull, T>(plan, tiles, fg, FG_FULL, plan->dtab_full, io, prm, st);
-    launch_fused<true, typename CfgOf<T>::Wide, T>(plan, tiles, fg, FG_FACE, plan->dtab_wide, io, prm, st);
+        launch_fused<true, CfgOf<float>::Wide, T>(plan, tiles, fg, FG_FACE, plan->dtab_wide, io, prm, st);
+    }
 }
 
 int run_fused(dgr_plan *plan, const StageIO &io, const RhsParams &prm, hipStream_t st) {
@@ -2890,7 +3041,7 @@ int dgr_plan_autotune(dgr_plan *plan, double *const *d_rhs, const double *const 
                 if (sch == SCH_FULL && p == 0) continue;
                 std::vector<std::vector<Tile>> per[NFGROUP];
                 for (auto &v : per) v.resize(ns);
-                for (size_t i = 0; i < ns; i++) block_tiles(plan->hblocks[kv.second[i]], kv.second[i], sch, per, i);
+                for (size_t i = 0; i < ns; i++) block_tiles(plan->hblocks[kv.second[i]], kv.second[i], p, sch, per, i);
                 std::vector<Tile> tiles;
                 int fg[NFGROUP + 1];
                 group_tiles(per, tiles, fg);
@@ -2923,6 +3074,7 @@ int dgr_plan_autotune(dgr_plan *plan, double *const *d_rhs, const double *const 
             plan->tiling[p][kv.first] = best;
         }
         HIP_OK(build_ftiles(plan, p));
+        if (!p) HIP_OK(build_ftiles(plan, LIST_CONS));
         if (plan->rk4_exec) {  // the captured step used the previous tile list
             HIP_OK(hipGraphExecDestroy(plan->rk4_exec));
             plan->rk4_exec = nullptr;
@@ -2948,6 +3100,7 @@ int dgr_plan_set_tiling(dgr_plan *plan, int precision, uint32_t nx, uint32_t ny,
     plan->tiling[p][{(int)nx, (int)ny, (int)nz}] = scheme;
     HIP_OK(hipSetDevice(plan->device));
     HIP_OK(build_ftiles(plan, p));
+    if (!p) HIP_OK(build_ftiles(plan, LIST_CONS));
     if (plan->rk4_exec) {  // the captured step used the previous tile list
         HIP_OK(hipGraphExecDestroy(plan->rk4_exec));
         plan->rk4_exec = nullptr;
@@ -3383,6 +3536,10 @@ int launch_padding_refresh(dgr_plan *plan, const VarPtrs &u, hipStream_t st) {
     return rc;
 }
 
+// Points per variable the HALO kernels serve: their 32-bit byte offsets, less a
+// few at the top that mean "read nothing" (StreamCtx::NOWHERE_AT_ALL).
+constexpr uint64_t HALO_POINTS_MAX = (1ull << 29) - 16;
+
 // With the padding refresh on, stages read linked padding straight from the
 // neighbours (k_fused<..., HALO>); plans whose variables hold 2^29 points or
 // more get the padding copied in by k_halo_fill before each stage instead.
@@ -3393,7 +3550,7 @@ bool halo_in_kernel(const dgr_plan *plan) {
         const char *e = std::getenv("DGR_HALO_IN_KERNEL");
         return !(e && std::string(e) == "0");
     }();
-    return plan->halo && plan->szpdof < (1ull << 29) && allowed;
+    return plan->halo && plan->szpdof < HALO_POINTS_MAX && allowed;
 }
 
 // The four stage launches of one RK4 step on the fused path (rkBSSN.cpp:764-860):
@@ -3830,8 +3987,8 @@ int dgr_constraints(dgr_plan *plan, double *d_ham, double *const *d_mom, double 
         StageIO io{};
         io.src = u;
         io.stage = -1;
-        const Tile *tiles = plan->d_ftiles[0];
-        const int *fg = plan->fgroup[0];
+        const Tile *tiles = plan->d_ftiles[LIST_CONS];
+        const int *fg = plan->fgroup[LIST_CONS];
         int n = fg[FG_WIDE + 1] - fg[FG_WIDE];
         if (n)
             hipLaunchKernelGGL((k_cons_fused<false, CfgWide>), dim3(n), dim3(CfgWide::FT), 0, st, io, o,

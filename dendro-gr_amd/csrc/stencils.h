@@ -112,6 +112,7 @@ __device__ __forceinline__ T ko(const T *s, int st, int a, int n, bool lo, bool 
 template <typename T>
 struct AxisConstsT {
     T d1_12, d1_60, d2_12, d2_180, ko_pre, ko_s3, ko_s2, ko_s1;
+    T ko_r3, ko_r2, ko_r1;  // 1/ko_s3 ..: a division by a block constant is ~30 instructions in FP64
 };
 using AxisConsts = AxisConstsT<double>;
 
@@ -128,6 +129,9 @@ __host__ __device__ inline AxisConsts axis_consts(double h) {
     k.ko_s3 = 59.0 / 48.0 * 64 * h;
     k.ko_s2 = 43.0 / 48.0 * 64 * h;
     k.ko_s1 = 49.0 / 48.0 * 64 * h;
+    k.ko_r3 = 1.0 / k.ko_s3;
+    k.ko_r2 = 1.0 / k.ko_s2;
+    k.ko_r1 = 1.0 / k.ko_s1;
     return k;
 }
 
@@ -203,5 +207,62 @@ __device__ __forceinline__ T ko_edge(const T *s, T r, int a, int ie, bool lo, bo
     return r;
 }
 #undef U
+
+// The interior formulas on taps already read: t[0..5] = U(-3) U(-2) U(-1) U(1)
+// U(2) U(3), c = U(0). Same terms, same order.
+struct Taps {
+    double t[6];
+};
+template <int ST>
+__device__ __forceinline__ Taps taps(const double *s) {
+    return {{s[-3 * ST], s[-2 * ST], s[-ST], s[ST], s[2 * ST], s[3 * ST]}};
+}
+__device__ __forceinline__ double d1_of(const Taps &a, double by60) {
+#pragma clang fp contract(off)
+    return (-a.t[0] + 9.0 * a.t[1] - 45.0 * a.t[2] + 45.0 * a.t[3] - 9.0 * a.t[4] + a.t[5]) * by60;
+}
+__device__ __forceinline__ double d2_of(const Taps &a, double c, double by180) {
+#pragma clang fp contract(off)
+    return (2.0 * a.t[0] - 27.0 * a.t[1] + 270.0 * a.t[2] - 490.0 * c + 270.0 * a.t[3] - 27.0 * a.t[4] + 2.0 * a.t[5]) * by180;
+}
+// The closures of a flagged face on the six values next to it along the axis,
+// e[0] on the face's node, for the point at distance l from the face (l > 2: r,
+// the interior value). All three rows are evaluated and one selected: every
+// lane reads the same six values' places, and no lane waits for another row's
+// loads. HI: the high face (its rows sum in another order, as the reference's).
+template <bool HI>
+__device__ __forceinline__ double d1_face(const double *e, double r, int l, double by12) {
+#pragma clang fp contract(off)
+    const double a = HI ? (3.0 * e[4] - 16.0 * e[3] + 36.0 * e[2] - 48.0 * e[1] + 25.0 * e[0]) * by12
+                        : (-25.0 * e[0] + 48.0 * e[1] - 36.0 * e[2] + 16.0 * e[3] - 3.0 * e[4]) * by12;
+    const double b = HI ? (-e[4] + 6.0 * e[3] - 18.0 * e[2] + 10.0 * e[1] + 3.0 * e[0]) * by12
+                        : (-3.0 * e[0] - 10.0 * e[1] + 18.0 * e[2] - 6.0 * e[3] + e[4]) * by12;
+    const double c = HI ? (e[4] - 8.0 * e[3] + 8.0 * e[1] - e[0]) * by12 : (e[0] - 8.0 * e[1] + 8.0 * e[3] - e[4]) * by12;
+    return l == 0 ? a : l == 1 ? b : l == 2 ? c : r;
+}
+template <bool HI>
+__device__ __forceinline__ double d2_face(const double *e, double r, int l, double by12) {
+#pragma clang fp contract(off)
+    const double a =
+        HI ? (-10.0 * e[5] + 61.0 * e[4] - 156.0 * e[3] + 214.0 * e[2] - 154.0 * e[1] + 45.0 * e[0]) * by12
+           : (45.0 * e[0] - 154.0 * e[1] + 214.0 * e[2] - 156.0 * e[3] + 61.0 * e[4] - 10.0 * e[5]) * by12;
+    const double b = HI ? (e[5] - 6.0 * e[4] + 14.0 * e[3] - 4.0 * e[2] - 15.0 * e[1] + 10.0 * e[0]) * by12
+                        : (10.0 * e[0] - 15.0 * e[1] - 4.0 * e[2] + 14.0 * e[3] - 6.0 * e[4] + e[5]) * by12;
+    const double c = HI ? (-e[4] + 16.0 * e[3] - 30.0 * e[2] + 16.0 * e[1] - e[0]) * by12
+                        : (-e[0] + 16.0 * e[1] - 30.0 * e[2] + 16.0 * e[3] - e[4]) * by12;
+    return l == 0 ? a : l == 1 ? b : l == 2 ? c : r;
+}
+template <typename K>
+__device__ __forceinline__ double ko_face(const double *e, double r, int l, const K &k) {
+#pragma clang fp contract(off)
+    const double a = (e[3] - 3.0 * e[2] + 3.0 * e[1] - e[0]) * k.ko_r3;
+    const double b = (e[4] - 6.0 * e[3] + 12.0 * e[2] - 10.0 * e[1] + 3.0 * e[0]) * k.ko_r2;
+    const double c = (e[5] - 6.0 * e[4] + 15.0 * e[3] - 19.0 * e[2] + 12.0 * e[1] - 3.0 * e[0]) * k.ko_r1;
+    return l == 0 ? a : l == 1 ? b : l == 2 ? c : r;
+}
+__device__ __forceinline__ double ko_of(const Taps &a, double c, double pre) {
+#pragma clang fp contract(off)
+    return pre * (-a.t[0] + 6.0 * a.t[1] - 15.0 * a.t[2] + 20.0 * c - 15.0 * a.t[3] + 6.0 * a.t[4] - a.t[5]);
+}
 
 }  // namespace dgr

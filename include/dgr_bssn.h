@@ -103,8 +103,8 @@ const char *dgr_last_error(void);
 
 /* Validates the block table (sizes >= 13 per axis, blocks inside [0, szpdof)),
  * splits every block into tiles and orders the work for the device. The
- * default is the single-kernel path (tiles of at most 7 x 7 x 5 points, or
- * 7 x 7 x 7 in mixed precision, see DGR_TILING_*; no derivative workspace);
+ * default is the single-kernel path (tiles of at most 7 x 7 x 7 points, see
+ * DGR_TILING_*; no derivative workspace);
  * the environment variable DGR_KERNEL=split selects the
  * two-kernel path (tiles of at most 7^3 points; a derivative workspace of 162
  * doubles per point in chunks of DGR_CHUNK_POINTS points).
@@ -129,7 +129,8 @@ int dgr_plan_set_precision(dgr_plan *plan, int precision);
 /* Tile shapes of the fused kernel (no counterpart in the reference, whose
  * kernels take fixed shapes). Every block is cut into columns of at most 7 x 7
  * points in x and y; along z a block without flagged faces is cut by one of:
- *   DGR_TILING_WT    parts of 5, a 1-2 point remainder in 128-thread tiles
+ *   DGR_TILING_WT    parts of 5, a 1-2 point remainder in 128-thread tiles (mixed
+ *                    precision) or in one tile with the 5 before it (FP64)
  *   DGR_TILING_W     near-equal parts of at most 5
  *   DGR_TILING_FULL  near-equal parts of at most 7 (384-thread tiles; mixed
  *                    precision only)
@@ -185,7 +186,9 @@ int dgr_plan_move_block(dgr_plan *plan, uint32_t b, uint64_t offset, const doubl
  * 1 equations, 2 boundary faces (the split path); 3 fused kernel on regular
  * tiles of blocks without flagged faces, 4 on thin tiles, 5 on tiles of
  * blocks with flagged faces, 6 the mixed-precision kernel on 7 x 7 x 7 tiles
- * of blocks without flagged faces (it replaces 3 and 4 in that precision). */
+ * of blocks without flagged faces (it replaces 3 and 4 in that precision).
+ * An FP64 launch on tiles of a regular part with its 1-2 point remainder counts
+ * in 3 and in 4, its time divided by the points of the two. */
 #define DGR_TIMING_KINDS 7
 int dgr_plan_set_timing(dgr_plan *plan, int enable);
 int dgr_plan_kernel_times(dgr_plan *plan, double *ms, int64_t *launches);
@@ -295,7 +298,7 @@ int dgr_rk45_step(dgr_plan *plan, double *const *d_u, double *dt, double tol, co
  * dgr_rk4_step(s) see its input state's padding refreshed, as the
  * reference's unzip between stages does (rkBSSN.cpp:764-860):
  * DGR_REFRESH_LINKED from same-level neighbours (the stage kernels of both
- * precisions read that padding from the neighbours when szpdof is below 2^29;
+ * precisions read that padding from the neighbours when szpdof is below 2^29 - 16;
  * larger plans copy it in before each stage), DGR_REFRESH_FULL also the rest
  * (written into the stage input before each stage). When the call returns, the caller's padding
  * is refreshed from the new interiors the same way. DGR_REFRESH_OFF (the
