@@ -1307,19 +1307,84 @@ __global__ __launch_bounds__(C::FT, 1) void k_cons_fused(const StageIO io, ConsP
         if (o.c[i]) o.c[i][idx] = (i >= 4 && axis) ? 0.0 : out.v[i];
 }
 
-// Copies the padding points of every block of src into dst (one workgroup per
-// block and variable): the RK4 work state's padding, refreshed from u once per
-// call of the RK4 entry points (u's padding is frozen while they run).
-__global__ __launch_bounds__(256) void k_pad_copy(VarPtrs dst, VarPtrs src, const DBlock *__restrict__ blocks) {
+// The q-th padding point of a block of nx x ny x nz points, in storage order:
+// the low planes, then per interior plane its low rows with the first
+// interior row's low end, the rows' ends two by two (high end and the next
+// row's low end lie together), the high rows, and the high planes.
+__device__ __forceinline__ int padding_point(int q, int nx, int ny, int nz) {
+    const int plane = nx * ny, mx = nx - 2 * PW, my = ny - 2 * PW;
+    if (q < PW * plane) return q;
+    const int per = plane - mx * my, k = (q - PW * plane) / per;  // interior plane and place in it
+    if (k >= nz - 2 * PW) return q + (nz - 2 * PW) * mx * my;
+    int r = q - PW * plane - k * per;
+    const int head = PW * nx + PW;
+    if (r >= head) r += mx * min((r - head) / (2 * PW) + 1, my);
+    return (PW + k) * plane + r;
+}
+
+// The RK4 work state's padding, set from u once per call of the RK4 entry
+// points (u's padding is frozen while they run).
+//
+// Without the padding refresh: whole blocks of src into dst, one workgroup per
+// block and variable. The interior goes along (stage 0 overwrites it): the rows'
+// ends alone are 48-byte pieces of lines that the memory has to merge, and
+// copying a third more bytes in whole lines is faster. 4096 blocks of 13^3 607
+// us against 817 for the padding alone (5.7 TB/s); 30 M points of uneven octree
+// 7.7 ms against 10.25.
+constexpr int COPY_UNROLL = 4;  // loads in flight per thread
+__global__ __launch_bounds__(256) void k_block_copy(VarPtrs dst, VarPtrs src, const DBlock *__restrict__ blocks) {
     const DBlock &B = blocks[blockIdx.x];
-    const int nx = B.n[0], ny = B.n[1], nz = B.n[2];
-    const int n = nx * ny * nz;
+    const int n = B.n[0] * B.n[1] * B.n[2];
     const double *__restrict__ s = src.p[blockIdx.y] + B.offset;
     double *__restrict__ d = dst.p[blockIdx.y] + B.offset;
-    for (int p = threadIdx.x; p < n; p += blockDim.x) {
-        const int i = p % nx, j = (p / nx) % ny, k = p / (nx * ny);
-        const bool inner = i >= PW && i < nx - PW && j >= PW && j < ny - PW && k >= PW && k < nz - PW;
-        if (!inner) d[p] = s[p];
+    for (int p0 = threadIdx.x; p0 < n; p0 += 256 * COPY_UNROLL) {
+        double t[COPY_UNROLL];
+#pragma unroll
+        for (int c = 0; c < COPY_UNROLL; c++)
+            if (p0 + 256 * c < n) t[c] = s[p0 + 256 * c];
+#pragma unroll
+        for (int c = 0; c < COPY_UNROLL; c++)
+            if (p0 + 256 * c < n) d[p0 + 256 * c] = t[c];
+    }
+}
+
+// With it: only padding that no neighbour supplies (stages read linked padding
+// from the neighbours, or refreshed before the stage), that is at level jumps
+// and the domain boundary. Of that, what a stage reads: a variable without
+// second derivatives is read on the sides of its block's interior only, one
+// with mixed derivatives along the edges too; the corners only with `corners`
+// (the mixed-precision kernels take their staging offset there). One thread per
+// point and all variables, a workgroup every gridDim.y-th chunk of 256 padding
+// points of a block. 4096 linked blocks of 13^3 848 -> 130 us, a refined octree
+// of 13560 blocks 2865 -> 557 us.
+__global__ __launch_bounds__(256) void k_pad_copy(VarPtrs dst, VarPtrs src, const DBlock *__restrict__ blocks,
+                                                  const int *__restrict__ nbr, int corners) {
+    __shared__ int s_linked[27];
+    const DBlock &B = blocks[blockIdx.x];
+    const int nx = B.n[0], ny = B.n[1], nz = B.n[2];
+    const bool mine = threadIdx.x < 27;
+    const int linked = mine ? nbr[27 * (size_t)blockIdx.x + threadIdx.x] >= 0 || threadIdx.x == 13 : 1;
+    if (mine) s_linked[threadIdx.x] = linked;
+    if (__syncthreads_and(linked)) return;
+    const int n = nx * ny * nz - (nx - 2 * PW) * (ny - 2 * PW) * (nz - 2 * PW);
+    for (int q = blockIdx.y * 256 + threadIdx.x; q < n; q += gridDim.y * 256) {
+        const int p = padding_point(q, nx, ny, nz);
+        const int k = p / (nx * ny), r = p - k * (nx * ny), j = r / nx, i = r - j * nx;
+        const int di = i < PW ? -1 : (i >= nx - PW ? 1 : 0);
+        const int dj = j < PW ? -1 : (j >= ny - PW ? 1 : 0);
+        const int dk = k < PW ? -1 : (k >= nz - PW ? 1 : 0);
+        if (s_linked[(di + 1) + 3 * (dj + 1) + 9 * (dk + 1)]) continue;
+        const int outside = (di != 0) + (dj != 0) + (dk != 0);
+        if (outside == 3 && !corners) continue;
+        const size_t at = B.offset + p;
+        const bool all = outside == 1 || corners;
+        double t[NV];
+#pragma unroll
+        for (int v = 0; v < NV; v++)
+            if (d2slot(v) >= 0 || all) t[v] = src.p[v][at];
+#pragma unroll
+        for (int v = 0; v < NV; v++)
+            if (d2slot(v) >= 0 || all) dst.p[v][at] = t[v];
     }
 }
 
@@ -1330,43 +1395,51 @@ __global__ __launch_bounds__(256) void k_pad_copy(VarPtrs dst, VarPtrs src, cons
 // is b's minus d*(n-2*PW-1) along each axis; every source is an interior point
 // and every destination a padding point, so blocks can be filled in place in
 // any order. nbr: 27 entries per block, -1 for none (that padding is kept).
-// One thread per point, one workgroup per 256-point chunk of a block
-// (blockIdx.x = chunk * nblocks + block: consecutive workgroups take the same
-// chunk of consecutive blocks, which measured faster than a block's chunks
-// in a row): the
-// neighbours' offsets are staged in LDS, and each padding point's index
-// arithmetic is done once for all 24 variables, whose loads are issued
-// together before the stores.
+// One thread per padding point and half of the variables, one workgroup per 256
+// of a block's points: the index arithmetic is done once for 12 variables,
+// whose loads are issued together before the stores (1, 4, 12, 24 variables
+// a thread: 8.56, 5.47, 5.21, 5.84 ms on the octree below). Workgroup w takes
+// entry (w % 8) * per + w / 8 of the list: workgroups are dealt round-robin to
+// the 8 XCDs, so each XCD walks a stretch of the list and neighbouring blocks
+// (in Morton order) find the interior nodes they share in one L2; the padding
+// itself is not read again and its stores are marked so. Bound by memory, with
+// rows' ends that are parts of lines: 49.0 M points of a refined octree of 30696
+// blocks of 13^3 6.62 -> 5.21 ms.
+constexpr int HALO_VARS = 12;
+static_assert(NV % HALO_VARS == 0, "whole groups of variables");
 __global__ __launch_bounds__(256) void k_halo_fill(VarPtrs u, const DBlock *__restrict__ blocks,
-                                                   const int *__restrict__ nbr, const int2 *__restrict__ wgs) {
+                                                   const int *__restrict__ nbr, const int2 *__restrict__ wgs, int nwg,
+                                                   int per) {
     __shared__ int64_t s_off[27];
-    const int2 w = wgs[blockIdx.x];  // (block, chunk of 256 points)
+    const int at = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if (at >= nwg) return;
+    const int2 w = wgs[at];  // (block, chunk of 256 padding points)
     const int b = w.x, chunk = w.y;
     const DBlock &B = blocks[b];
     const int nx = B.n[0], ny = B.n[1], nz = B.n[2];
-    const int n = nx * ny * nz;
     if (threadIdx.x < 27) {
         const int nb = nbr[27 * (size_t)b + threadIdx.x];
         s_off[threadIdx.x] = (nb >= 0 && threadIdx.x != 13) ? (int64_t)blocks[nb].offset : -1;
     }
     __syncthreads();
-    const int p = chunk * blockDim.x + threadIdx.x;
-    if (p < n) {
-        const int i = p % nx, j = (p / nx) % ny, k = p / (nx * ny);
-        const int di = i < PW ? -1 : (i >= nx - PW ? 1 : 0);
-        const int dj = j < PW ? -1 : (j >= ny - PW ? 1 : 0);
-        const int dk = k < PW ? -1 : (k >= nz - PW ? 1 : 0);
-        const int64_t off = s_off[(di + 1) + 3 * (dj + 1) + 9 * (dk + 1)];  // -1 for interior points too
-        if (off < 0) return;
-        const int si = i - di * (nx - 2 * PW - 1), sj = j - dj * (ny - 2 * PW - 1), sk = k - dk * (nz - 2 * PW - 1);
-        const size_t src = (size_t)off + si + (size_t)nx * (sj + (size_t)ny * sk);
-        const size_t dst = B.offset + p;
-        double t[NV];
+    const int q = chunk * 256 + threadIdx.x;
+    if (q >= nx * ny * nz - (nx - 2 * PW) * (ny - 2 * PW) * (nz - 2 * PW)) return;
+    const int p = padding_point(q, nx, ny, nz);
+    const int k = p / (nx * ny), r = p - k * (nx * ny), j = r / nx, i = r - j * nx;
+    const int di = i < PW ? -1 : (i >= nx - PW ? 1 : 0);
+    const int dj = j < PW ? -1 : (j >= ny - PW ? 1 : 0);
+    const int dk = k < PW ? -1 : (k >= nz - PW ? 1 : 0);
+    const int64_t off = s_off[(di + 1) + 3 * (dj + 1) + 9 * (dk + 1)];
+    if (off < 0) return;
+    const int si = i - di * (nx - 2 * PW - 1), sj = j - dj * (ny - 2 * PW - 1), sk = k - dk * (nz - 2 * PW - 1);
+    const size_t src = (size_t)off + si + (size_t)nx * (sj + (size_t)ny * sk);
+    const size_t dst = B.offset + p;
+    const int v0 = blockIdx.y * HALO_VARS;
+    double t[HALO_VARS];
 #pragma unroll
-        for (int v = 0; v < NV; v++) t[v] = u.p[v][src];
+    for (int v = 0; v < HALO_VARS; v++) t[v] = u.p[v0 + v][src];
 #pragma unroll
-        for (int v = 0; v < NV; v++) u.p[v][dst] = t[v];
-    }
+    for (int v = 0; v < HALO_VARS; v++) __builtin_nontemporal_store(t[v], &u.p[v0 + v][dst]);
 }
 
 // The rest of the padding refresh (the interpolating part of unzip,
@@ -3163,7 +3236,11 @@ int launch_pad_copy(dgr_plan *plan, const RkBuffers &buf, const VarPtrs &u, hipS
     if (!nb) return DGR_OK;
     VarPtrs w;
     for (int v = 0; v < NV; v++) w.p[v] = buf.wstate + (size_t)v * plan->szpdof;
-    hipLaunchKernelGGL(k_pad_copy, dim3(nb, NV), dim3(256), 0, st, w, u, plan->d_blocks);
+    if (plan->halo)
+        hipLaunchKernelGGL(k_pad_copy, dim3(nb, 8), dim3(256), 0, st, w, u, plan->d_blocks, plan->d_nbr,
+                           plan->precision == DGR_PRECISION_MIXED ? 1 : 0);
+    else
+        hipLaunchKernelGGL(k_block_copy, dim3(nb, NV), dim3(256), 0, st, w, u, plan->d_blocks);
     HIP_OK(hipGetLastError());
     return DGR_OK;
 }
@@ -3232,23 +3309,21 @@ int link_neighbors(dgr_plan *plan) {
     if (nb) HIP_OK(hipMemcpy(plan->d_nbo, off.data(), sizeof(int64_t) * 27 * nb, hipMemcpyHostToDevice));
     plan->nlinks = links;
     plan->nfill = -1;  // the general fill records follow the links
-    // k_halo_fill's workgroups: (block, chunk of 256 points) for the blocks
-    // with at least one link, chunk-major (consecutive workgroups take
-    // different blocks)
+    // k_halo_fill's workgroups: (block, chunk of 256 padding points) for the
+    // blocks with at least one link
     std::vector<int2> wgs;
-    int maxch = 0;
     std::vector<int> nch(nb, 0);
     for (size_t b = 0; b < nb; b++) {
         bool linked = false;
         for (int d = 0; d < 27 && !linked; d++) linked = plan->hnbr[27 * b + d] >= 0;
         const DBlock &B = plan->hblocks[b];
-        if (linked) nch[b] = (int)(((int64_t)B.n[0] * B.n[1] * B.n[2] + 255) / 256);
-        maxch = std::max(maxch, nch[b]);
+        const int64_t pad = (int64_t)B.n[0] * B.n[1] * B.n[2] -
+                            (int64_t)(B.n[0] - 2 * PW) * (B.n[1] - 2 * PW) * (B.n[2] - 2 * PW);
+        if (linked) nch[b] = (int)((pad + 255) / 256);
     }
-    for (int c = 0; c < maxch; c++)
-        for (size_t b = 0; b < nb; b++)
-            if (c < nch[b]) wgs.push_back(make_int2((int)b, c));
-    if (wgs.size() > (size_t)INT32_MAX) return fail(DGR_E_INVALID, "padding fill: too many blocks x points");
+    for (size_t b = 0; b < nb; b++)
+        for (int c = 0; c < nch[b]; c++) wgs.push_back(make_int2((int)b, c));
+    if (wgs.size() > (size_t)INT32_MAX - 8) return fail(DGR_E_INVALID, "padding fill: too many blocks x points");
     if (plan->rk4_exec && plan->halo) {  // a captured step with the refresh holds the old table
         HIP_OK(hipGraphExecDestroy(plan->rk4_exec));
         plan->rk4_exec = nullptr;
@@ -3522,8 +3597,9 @@ int launch_fill_general(dgr_plan *plan, const VarPtrs &u, hipStream_t st) {
 
 int launch_halo_fill(dgr_plan *plan, const VarPtrs &u, hipStream_t st) {
     if (plan->nhalo_wg <= 0) return DGR_OK;
-    hipLaunchKernelGGL(k_halo_fill, dim3((uint32_t)plan->nhalo_wg), dim3(256), 0, st, u, plan->d_blocks, plan->d_nbr,
-                       plan->d_halo_wg);
+    const int per = (int)((plan->nhalo_wg + 7) / 8);
+    hipLaunchKernelGGL(k_halo_fill, dim3(8u * (uint32_t)per, NV / HALO_VARS), dim3(256), 0, st, u, plan->d_blocks, plan->d_nbr,
+                       plan->d_halo_wg, (int)plan->nhalo_wg, per);
     HIP_OK(hipGetLastError());
     return DGR_OK;
 }
