@@ -2985,7 +2985,8 @@ void launch_fused(dgr_plan *plan, const Tile *tiles, const int *fg, int group, i
                   const RhsParams &prm, hipStream_t st) {
     const int n = fg[group + 1] - fg[group];
     if (!n) return;
-    // the kernel's parameters, in order (StreamIO holds the RhsParams)
+    // the kernel's parameters, in order (k_stream: without the RhsParams, which
+    // StreamIO holds, and the slot table)
     constexpr bool FP64 = sizeof(T) == sizeof(double);
     std::conditional_t<FP64, StreamIO, StageIO> a_io;
     if constexpr (FP64) a_io = stream_io(io, prm);

@@ -230,14 +230,21 @@ __device__ __forceinline__ double d2_of(const Taps &a, double c, double by180) {
 // the interior value). All three rows are evaluated and one selected: every
 // lane reads the same six values' places, and no lane waits for another row's
 // loads. HI: the high face (its rows sum in another order, as the reference's).
+template <bool HI, int L>
+__device__ __forceinline__ double d1_row(const double *e, double by12) {
+#pragma clang fp contract(off)
+    if constexpr (L == 0)
+        return HI ? (3.0 * e[4] - 16.0 * e[3] + 36.0 * e[2] - 48.0 * e[1] + 25.0 * e[0]) * by12
+                  : (-25.0 * e[0] + 48.0 * e[1] - 36.0 * e[2] + 16.0 * e[3] - 3.0 * e[4]) * by12;
+    else if constexpr (L == 1)
+        return HI ? (-e[4] + 6.0 * e[3] - 18.0 * e[2] + 10.0 * e[1] + 3.0 * e[0]) * by12
+                  : (-3.0 * e[0] - 10.0 * e[1] + 18.0 * e[2] - 6.0 * e[3] + e[4]) * by12;
+    else
+        return HI ? (e[4] - 8.0 * e[3] + 8.0 * e[1] - e[0]) * by12 : (e[0] - 8.0 * e[1] + 8.0 * e[3] - e[4]) * by12;
+}
 template <bool HI>
 __device__ __forceinline__ double d1_face(const double *e, double r, int l, double by12) {
-#pragma clang fp contract(off)
-    const double a = HI ? (3.0 * e[4] - 16.0 * e[3] + 36.0 * e[2] - 48.0 * e[1] + 25.0 * e[0]) * by12
-                        : (-25.0 * e[0] + 48.0 * e[1] - 36.0 * e[2] + 16.0 * e[3] - 3.0 * e[4]) * by12;
-    const double b = HI ? (-e[4] + 6.0 * e[3] - 18.0 * e[2] + 10.0 * e[1] + 3.0 * e[0]) * by12
-                        : (-3.0 * e[0] - 10.0 * e[1] + 18.0 * e[2] - 6.0 * e[3] + e[4]) * by12;
-    const double c = HI ? (e[4] - 8.0 * e[3] + 8.0 * e[1] - e[0]) * by12 : (e[0] - 8.0 * e[1] + 8.0 * e[3] - e[4]) * by12;
+    const double a = d1_row<HI, 0>(e, by12), b = d1_row<HI, 1>(e, by12), c = d1_row<HI, 2>(e, by12);
     return l == 0 ? a : l == 1 ? b : l == 2 ? c : r;
 }
 template <bool HI>

@@ -47,10 +47,13 @@ struct SCfg {
     static constexpr int all(bool halo) { return cross(halo) + NONE * (pairs(halo) - 4) + NOUT * 4; }
     static constexpr int passes(bool halo) { return (all(halo) + FT - 1) / FT; }
     static constexpr int cross_passes(bool halo) { return (cross(halo) + FT - 1) / FT; }
-    static constexpr int NDX = TMAX * (RMAX * FZ + TMAX * 2 * PW);
-    static constexpr int NDY = TMAX * TMAX * (FZ + 2 * PW);
-    static constexpr int DXIT = (NDX + FT - 1) / FT;
-    static constexpr int DYIT = (NDY + FT - 1) / FT;
+    // D_x is evaluated along whole x rows of 7 points, D_y along whole y columns,
+    // one a thread: D_y(D_x u) reads D_x on the tile's z planes (all region rows),
+    // D_z(D_x u) on its y rows (all region planes). The first XWAVES waves take the
+    // rows, the others the columns.
+    static constexpr int XLINES = RMAX * FZ + TMAX * 2 * PW, YLINES = TMAX * (FZ + 2 * PW);
+    static constexpr int XWAVES = (XLINES + 63) / 64;
+    static_assert(YLINES <= FT - 64 * XWAVES, "a thread per line");
     static constexpr int NSDX = TMAX + FRX * (RMAX - 1) + FRXY * (FZ + 2 * PW - 1);
     static constexpr int NSDY = TMAX + FRX * (TMAX - 1) + FRXY * (FZ + 2 * PW - 1);
     static constexpr int RB = DEEP ? 3 : 2, DB = DEEP ? 2 : 1;
@@ -83,7 +86,7 @@ struct StreamIO {
 
 template <bool FACE, class C, bool HALO, bool GAUGE>
 struct StreamCtx {
-    static constexpr int FT = C::FT, NBUF = C::NBUF, DXIT = C::DXIT, DYIT = C::DYIT;
+    static constexpr int FT = C::FT, NBUF = C::NBUF;
     static constexpr int PASS = C::passes(HALO), CROSS = C::cross_passes(HALO);
     // Variables in flight (1 to 3) once variable Q is staged, that is while phase
     // Q runs (one to three in the later phases measured the same to 1%)
@@ -126,7 +129,9 @@ struct StreamCtx {
     uint32_t goff[PASS], goff_cross, spot[(PASS + 1) / 2];
     typedef double Pair __attribute__((ext_vector_type(2)));
     Pair pre[3][PASS];
-    uint32_t dw[DXIT > DYIT ? DXIT : DYIT];  // D_x slot | D_y slot << 16
+    int line;        // where this thread's D_x row or D_y column starts in the region
+    bool has_line;
+    bool x_wave;     // (uniform) this wave's lines are rows
     // the current phase
     double d1[3], d2[6], kv, centre;
     // the stage update
@@ -193,6 +198,46 @@ struct StreamCtx {
 #pragma unroll
         for (int k = 0; k < N; k++) e[k] = p[(HI ? -k : k) * stride<A>()];
     }
+    // First derivatives of the tile's (up to 7) points along axis A from the 13
+    // region values of the line at s: 13 LDS reads for 7 results, where a
+    // stencil at a time reads 42
+    template <int A>
+    __device__ __forceinline__ void d1_line(const double *s, double *to) const {
+        constexpr int ST = stride<A>();
+        double u[RMAX], r[TMAX];
+#pragma unroll
+        for (int k = 0; k < RMAX; k++) u[k] = s[k * ST];
+#pragma unroll
+        for (int i = 0; i < TMAX; i++)
+            r[i] = dgr::d1_of({{u[i], u[i + 1], u[i + 2], u[i + 4], u[i + 5], u[i + 6]}}, kc[A]);
+        if constexpr (FACE) {
+            const double by12 = K[A].d1_12;
+            if (lo<A>()) {
+                r[0] = dgr::d1_row<false, 0>(u + PW, by12);
+                r[1] = dgr::d1_row<false, 1>(u + PW, by12);
+                r[2] = dgr::d1_row<false, 2>(u + PW, by12);
+            }
+            if (hi<A>()) {
+                // the last point's place is the tile's extent (4 to 7) less one
+                auto at_end = [&](auto last) {
+                    constexpr int N = decltype(last)::value;
+                    const double e[5] = {u[PW + N], u[PW + N - 1], u[PW + N - 2], u[PW + N - 3], u[PW + N - 4]};
+                    r[N] = dgr::d1_row<true, 0>(e, by12);
+                    r[N - 1] = dgr::d1_row<true, 1>(e, by12);
+                    r[N - 2] = dgr::d1_row<true, 2>(e, by12);
+                };
+                switch (last_point<A>()) {
+                    case 3: at_end(std::integral_constant<int, 3>()); break;
+                    case 4: at_end(std::integral_constant<int, 4>()); break;
+                    case 5: at_end(std::integral_constant<int, 5>()); break;
+                    default: at_end(std::integral_constant<int, 6>());
+                }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < TMAX; i++) to[i * ST] = r[i];
+    }
+
     // N first derivatives along axis A from their taps; s: where they were read,
     // l: the points' places within the tile along A (a tile with lo<A>() starts
     // on that face, one with hi<A>() ends on it). The closures of all N in one
@@ -273,36 +318,13 @@ struct StreamCtx {
             centre = s[0];
         };
         if constexpr (MIXED) {
-            // D_x on tile-x x region-y x region-z, D_y on tile-x x tile-y x region-z: the mixed
-            // derivatives are D_y(D_x u), D_z(D_x u), D_z(D_y u); slots beyond
-            // the tile read valid LDS and land where nobody reads
-            dgr::Taps gx[DXIT], gy[DYIT];
-#pragma unroll
-            for (int it = 0; it < DXIT; it++) gx[it] = dgr::taps<1>(t + (dw[it] & 0xffffu) + PW);
-#pragma unroll
-            for (int it = 0; it < DYIT; it++) gy[it] = dgr::taps<FRX>(t + (dw[it] >> 16) + PW + FRX * PW);
-            const double *at[DXIT > DYIT ? DXIT : DYIT];
-            int l[DXIT > DYIT ? DXIT : DYIT];
-            double r[DXIT > DYIT ? DXIT : DYIT];
-#pragma unroll
-            for (int it = 0; it < DXIT; it++) {
-                const int w = dw[it] & 0xffffu;
-                at[it] = t + w + PW;
-                l[it] = FACE ? w % FRX : 0;
-            }
-            D1<0, DXIT>(gx, at, l, r);
-#pragma unroll
-            for (int it = 0; it < DXIT; it++) dx[dw[it] & 0xffffu] = r[it];
+            // the mixed derivatives are D_y(D_x u), D_z(D_x u), D_z(D_y u)
             own();
-#pragma unroll
-            for (int it = 0; it < DYIT; it++) {
-                const int w = dw[it] >> 16;
-                at[it] = t + w + PW + FRX * PW;
-                l[it] = FACE ? (w / FRX) % FRX : 0;
+            if (x_wave) {
+                if (has_line) d1_line<0>(t + line, dx + line);
+            } else {
+                if (has_line) d1_line<1>(t + line + PW, dy + line);
             }
-            D1<1, DYIT>(gy, at, l, r);
-#pragma unroll
-            for (int it = 0; it < DYIT; it++) dy[dw[it] >> 16] = r[it];
         } else {
             own();
         }
@@ -513,7 +535,7 @@ template <bool FACE, class C, bool HALO, bool GAUGE>
 __global__ __launch_bounds__(C::FT, 2) void k_stream(const StreamIO io, const DBlock *__restrict__ blocks,
                                                      const dgr::AxisConsts *__restrict__ bconst,
                                                      const Tile *__restrict__ tiles,
-                                                     const uint16_t *__restrict__ tabs, int dtab) {
+                                                     const uint16_t *__restrict__ tabs) {
     __shared__ double s_tile[C::RB * C::NBUF];
     __shared__ double s_dx[C::DB * C::NSDX];
     __shared__ double s_dy[C::DB * C::NSDY];
@@ -608,10 +630,21 @@ __global__ __launch_bounds__(C::FT, 2) void k_stream(const StreamIO io, const DB
     c.lq = c.active ? ((uint32_t)tl.q0 + tabs[tl.lanetab + C::FT + tid]) * (uint32_t)sizeof(double) : c.NOWHERE;
     c.face = FACE && ((c.lox && lx == 0) || (c.hix && lx == ex - 1) || (c.loy && ly == 0) || (c.hiy && ly == ey - 1) ||
                       (c.loz && lz == 0) || (c.hiz && lz == ez - 1));
-#pragma unroll
-    for (int it = 0; it < (C::DXIT > C::DYIT ? C::DXIT : C::DYIT); it++)
-        c.dw[it] = (it < C::DXIT ? (uint32_t)tabs[dtab + it * C::FT + tid] : 0u) |
-                   (it < C::DYIT ? (uint32_t)tabs[dtab + (C::DXIT + it) * C::FT + tid] << 16 : 0u);
+    // this thread's line: D_x rows first on the tile's z planes (all 13 of each),
+    // then on its y rows of the other planes
+    {
+        c.x_wave = __builtin_amdgcn_readfirstlane(tid >> 6) < C::XWAVES;
+        const int l = c.x_wave ? tid : tid - 64 * C::XWAVES;
+        c.has_line = l < (c.x_wave ? C::XLINES : C::YLINES);
+        if (c.x_wave) {
+            const int o = l - RMAX * C::FZ, q = o / TMAX;
+            const int kk = o < 0 ? PW + l / RMAX : q < PW ? q : q + C::FZ;
+            const int jj = o < 0 ? l % RMAX : PW + o - TMAX * q;
+            c.line = FRX * jj + FRXY * kk;
+        } else {
+            c.line = l % TMAX + FRXY * (l / TMAX);
+        }
+    }
     // sigma: sqrt(chi) * eps (rhs.cpp:356-360), or one number
     c.root = 1.0;
     c.eps_gauge = c.eps_other = io.prm.ko_sigma;
