@@ -1725,20 +1725,37 @@ __device__ __forceinline__ bool owned_elsewhere(const int *__restrict__ nbr, int
     return false;
 }
 
+// One launch over all chunks (a workgroup finds its chunk by bisection, in
+// scalar registers), where a launch per chunk of 512 workgroups took 8.8 us
+// each, two workgroups a CU and a drain between them: 36 chunks (4.6 M points)
+// 310 -> 74 us, the constraints with their norm 2.32 -> 2.06 ms. What is left is
+// the read of c's interior rows (56 bytes of each 104-byte row). The sum of a workgroup keeps
+// the order of a tree over 256 values halved from the top, which the first
+// wave can finish by itself after one exchange through LDS.
 __global__ __launch_bounds__(NTHREADS) void k_norm_partial(const double *__restrict__ c, NormMask m,
                                                           const DBlock *__restrict__ blocks,
                                                           const Tile *__restrict__ tiles,
-                                                          const int *__restrict__ wg_tile, int tile_end, int64_t P,
+                                                          const int *__restrict__ wg_tile,
+                                                          const Chunk *__restrict__ chunks, int nchunk, int first_wg,
                                                           const int *__restrict__ nbr, double *__restrict__ psum,
                                                           unsigned long long *__restrict__ pcnt) {
 #pragma clang fp contract(off)
+    static_assert(NTHREADS == 256, "the sum's tree");
     __shared__ double s_sum[NTHREADS];
-    __shared__ unsigned long long s_cnt[NTHREADS];
-    const int64_t q = (int64_t)blockIdx.x * NTHREADS + threadIdx.x;
+    __shared__ int s_cnt[NTHREADS / 64];
+    const int wg = first_wg + (int)blockIdx.x;
+    int lo = 0, hi = nchunk;  // the last chunk with wg_begin <= wg
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (chunks[mid].wg_begin <= wg) lo = mid;
+        else hi = mid;
+    }
+    const int tile_end = chunks[lo].tile_end;
+    const int64_t q = (int64_t)(wg - chunks[lo].wg_begin) * NTHREADS + threadIdx.x;
     double v2 = 0.0;
-    unsigned long long cnt = 0;
-    if (q < P) {
-        int t = wg_tile[blockIdx.x];
+    bool counts = false;
+    if (q < chunks[lo].npoints) {
+        int t = wg_tile[wg];
         while (t + 1 < tile_end && q >= tiles[t + 1].q0) t++;
         const Tile T = tiles[t];
         const DBlock B = blocks[T.block];
@@ -1753,22 +1770,21 @@ __global__ __launch_bounds__(NTHREADS) void k_norm_partial(const double *__restr
         if (!(d1 < m.r1 || d2 < m.r2) && !owned_elsewhere(nbr, T.block, g, B)) {
             const double v = c[g.idx];
             v2 = v * v;
-            cnt = 1;
+            counts = true;
         }
     }
-    s_sum[threadIdx.x] = v2;
-    s_cnt[threadIdx.x] = cnt;
+    const int n = __popcll(__ballot(counts));
+    const int t = threadIdx.x;
+    s_sum[t] = v2;
+    if ((t & 63) == 0) s_cnt[t >> 6] = n;
     __syncthreads();
-    for (int w = NTHREADS / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) {
-            s_sum[threadIdx.x] += s_sum[threadIdx.x + w];
-            s_cnt[threadIdx.x] += s_cnt[threadIdx.x + w];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        psum[blockIdx.x] = s_sum[0];
-        pcnt[blockIdx.x] = s_cnt[0];
+    if (t >= 64) return;
+    double a = (v2 + s_sum[t + 128]) + (s_sum[t + 64] + s_sum[t + 192]);
+#pragma unroll
+    for (int w = 32; w > 0; w >>= 1) a += __shfl_down(a, w, 64);
+    if (t == 0) {
+        psum[wg] = a;
+        pcnt[wg] = (unsigned long long)(s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3]);
     }
 }
 
@@ -2166,6 +2182,7 @@ struct dgr_plan {
     DBlock *d_blocks = nullptr;
     Tile *d_tiles = nullptr;
     int *d_wg_tile = nullptr;
+    Chunk *d_chunks = nullptr;  // `chunks`, for kernels that run over all of them
     int *d_face_tiles = nullptr;
     double *d_W = nullptr;
     int64_t max_chunk_points = 0;
@@ -2707,6 +2724,10 @@ int dgr_plan_create(int device, const dgr_block *blocks, uint32_t nblocks, uint6
     if (e == hipSuccess && nblocks) e = hipMalloc(&plan->d_blocks, sizeof(DBlock) * hb.size());
     if (e == hipSuccess && !tiles.empty()) e = hipMalloc(&plan->d_tiles, sizeof(Tile) * tiles.size());
     if (e == hipSuccess && !wg_tile.empty()) e = hipMalloc(&plan->d_wg_tile, sizeof(int) * wg_tile.size());
+    if (e == hipSuccess && !plan->chunks.empty()) {
+        e = hipMalloc(&plan->d_chunks, sizeof(Chunk) * plan->chunks.size());
+        if (e == hipSuccess) e = hipMemcpy(plan->d_chunks, plan->chunks.data(), sizeof(Chunk) * plan->chunks.size(), hipMemcpyHostToDevice);
+    }
     if (e == hipSuccess && !face_tiles.empty()) e = hipMalloc(&plan->d_face_tiles, sizeof(int) * face_tiles.size());
     if (e == hipSuccess) e = hipMalloc(&plan->d_tabs, sizeof(uint16_t) * tabs.size());
     if (e == hipSuccess) e = hipMemcpy(plan->d_tabs, tabs.data(), sizeof(uint16_t) * tabs.size(), hipMemcpyHostToDevice);
@@ -2743,6 +2764,7 @@ int dgr_plan_destroy(dgr_plan *plan) {
     (void)hipFree(plan->d_blocks);
     (void)hipFree(plan->d_tiles);
     (void)hipFree(plan->d_wg_tile);
+    (void)hipFree(plan->d_chunks);
     (void)hipFree(plan->d_face_tiles);
     (void)hipFree(plan->d_W);
     (void)hipFree(plan->d_stage);
@@ -4112,7 +4134,7 @@ int dgr_ham_constraint(dgr_plan *plan, double *d_ham, const double *const *d_u, 
 }  // extern "C"
 
 namespace {
-// The two norm kernels over every chunk: partials into psum/pcnt (one per
+// The two norm kernels: partials into psum/pcnt (one per
 // k_rhs-style workgroup, nwg_total of each), then the sum and count into
 // res[0..1] and, with d_norm, the norm into d_norm[0]. Linked neighbours
 // (when the table holds links) count each shared node once.
@@ -4123,10 +4145,11 @@ int launch_norm(dgr_plan *plan, const double *d_c, const double *bh, double r1, 
     m.r1 = r1;
     m.r2 = r2;
     const int *nbr = plan->nlinks > 0 ? plan->d_nbr : nullptr;
-    for (const Chunk &c : plan->chunks)
-        hipLaunchKernelGGL(k_norm_partial, dim3(c.nwg), dim3(NTHREADS), 0, st, d_c, m, plan->d_blocks, plan->d_tiles,
-                           plan->d_wg_tile + c.wg_begin, c.tile_end, (int64_t)c.npoints, nbr, psum + c.wg_begin,
-                           pcnt + c.wg_begin);
+    constexpr int MAX_WG = 1 << 23;  // a launch holds fewer than 2^32 threads
+    for (int w = 0; w < plan->nwg_total; w += MAX_WG)
+        hipLaunchKernelGGL(k_norm_partial, dim3(std::min(MAX_WG, plan->nwg_total - w)), dim3(NTHREADS), 0, st, d_c, m,
+                           plan->d_blocks, plan->d_tiles, plan->d_wg_tile, plan->d_chunks, (int)plan->chunks.size(), w,
+                           nbr, psum, pcnt);
     hipLaunchKernelGGL(k_norm_final, dim3(1), dim3(NTHREADS), 0, st, psum, pcnt, plan->nwg_total, res, d_norm);
     HIP_OK(hipGetLastError());
     return DGR_OK;
