@@ -36,12 +36,14 @@ def regenerate(verbose=False):
           os.path.join(HERE, "csrc", "bssn_rhs_generated.h")], verbose)
 
 
-# The library's three units, compiled from one source (they differ in what they
+# The library's four units, compiled from one source (they differ in what they
 # instantiate and in the instruction scheduling that measured faster): host
-# code with the diagnostics' kernels, the FP32 fused kernels, the FP64 stage kernels.
+# code with the diagnostics' kernels, the FP32 fused kernels, the FP64 stage kernels,
+# the FP64 stage kernel of small plans.
 UNITS = {"main": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
          "f32": ["-DDGR_F32_KERNELS"],
-         "stream": ["-DDGR_STREAM_KERNELS"]}
+         "stream": ["-DDGR_STREAM_KERNELS"],
+         "small": ["-DDGR_SMALL_KERNELS"]}
 
 
 def build_bssn(src: str, out: str, verbose: bool = False, extra=()) -> None:

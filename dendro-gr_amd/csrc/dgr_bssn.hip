@@ -2102,12 +2102,13 @@ int fail(int code, const std::string &msg) {
 }  // namespace
 
 #ifdef DGR_F32_KERNELS
-// The library compiles this source twice. With DGR_F32_KERNELS the unit holds
-// only the FP32 fused kernels and this table of their addresses: they are
-// built with the compiler's default instruction scheduler, while the main
-// unit (everything else, FP64 kernels included) is built with the iterative
-// ILP scheduler, which is 3% faster on the FP64 kernels and spills the FP32
-// ones (measured).
+// The library compiles this source four times. With DGR_F32_KERNELS the unit holds
+// only the FP32 fused kernels and this table of their addresses, with
+// DGR_STREAM_KERNELS only the FP64 stage kernels and theirs, with
+// DGR_SMALL_KERNELS the small plans'. These are built with the compiler's default
+// instruction scheduler, the main unit (everything else) with the iterative ILP
+// scheduler, which was 3% faster on the one-wave FP64 kernels (the constraints'
+// are left of those) and spills the FP32 ones (measured).
 extern "C" __attribute__((visibility("hidden"))) void dgr_internal_fused_f32_kernels(const void **k) {
     k[0] = reinterpret_cast<const void *>(&k_fused<false, CfgOf<float>::Wide, float>);
     k[1] = reinterpret_cast<const void *>(&k_fused<false, CfgOf<float>::Thin, float>);
@@ -2121,9 +2122,6 @@ extern "C" __attribute__((visibility("hidden"))) void dgr_internal_fused_f32_ker
 #elif defined(DGR_STREAM_KERNELS)
 // The FP64 stage kernels (stream_fp64.h), [halo][gauge][wide, full, face]
 extern "C" __attribute__((visibility("hidden"))) void dgr_internal_stream_kernels(const void **k) {
-#ifdef DGR_PROBE
-    k[0] = reinterpret_cast<const void *>(&DGR_PROBE);
-#else
     k[0] = reinterpret_cast<const void *>(&k_stream<false, SWide, false, false>);
     k[1] = reinterpret_cast<const void *>(&k_stream<false, SFull, false, false>);
     k[2] = reinterpret_cast<const void *>(&k_stream<true, SWide, false, false>);
@@ -2136,11 +2134,19 @@ extern "C" __attribute__((visibility("hidden"))) void dgr_internal_stream_kernel
     k[9] = reinterpret_cast<const void *>(&k_stream<false, SWide, true, true>);
     k[10] = reinterpret_cast<const void *>(&k_stream<false, SFull, true, true>);
     k[11] = reinterpret_cast<const void *>(&k_stream<true, SWide, true, true>);
-#endif
+}
+#elif defined(DGR_SMALL_KERNELS)
+// k_stream_small, [halo][gauge]
+extern "C" __attribute__((visibility("hidden"))) void dgr_internal_small_kernels(const void **k) {
+    k[0] = reinterpret_cast<const void *>(&k_stream_small<false, false>);
+    k[1] = reinterpret_cast<const void *>(&k_stream_small<false, true>);
+    k[2] = reinterpret_cast<const void *>(&k_stream_small<true, false>);
+    k[3] = reinterpret_cast<const void *>(&k_stream_small<true, true>);
 }
 #else
 extern "C" void dgr_internal_fused_f32_kernels(const void **k);
 extern "C" void dgr_internal_stream_kernels(const void **k);
+extern "C" void dgr_internal_small_kernels(const void **k);
 
 namespace {
 // Device scratch of dgr_constraint_l2_norm_noalloc: the norm's per-workgroup
@@ -3035,6 +3041,24 @@ void launch_fused(dgr_plan *plan, const Tile *tiles, const int *fg, int group, i
 template <bool HALO, bool GAUGE>
 void launch_stream(dgr_plan *plan, const Tile *tiles, const int *fg, const StageIO &io, const RhsParams &prm,
                    hipStream_t st) {
+    // At most a tile for each CU, of more than one kind: one launch (with timing
+    // on a launch a kind, so that each has its own time). Of one kind, or with
+    // more tiles, where two of the smaller workgroups share a CU: a launch a kind.
+    const int nface = fg[FG_FULL] - fg[FG_FACE], nfull = fg[NFGROUP] - fg[FG_FULL], n = fg[NFGROUP] - fg[FG_WIDE];
+    const int kinds = (n > nface + nfull) + (nface > 0) + (nfull > 0);
+    if (kinds > 1 && n <= SMALL_TILES && !plan->timing) {
+        static const void *const *tab = [] {
+            static const void *k[4];
+            dgr_internal_small_kernels(k);
+            return k;
+        }();
+        StreamIO a_io = stream_io(io, prm);
+        const Tile *a_tiles = tiles + fg[FG_WIDE];
+        int face0 = n - nface - nfull, full0 = n - nfull;
+        void *args[] = {&a_io, &plan->d_blocks, &plan->d_bconst, &a_tiles, &plan->d_tabs, &face0, &full0};
+        (void)hipLaunchKernel(tab[2 * HALO + GAUGE], dim3(n), dim3(SFull::FT), args, 0, st);
+        return;
+    }
     launch_fused<false, CfgWide, double, HALO, GAUGE>(plan, tiles, fg, FG_WIDE, plan->dtab_wide, io, prm, st);
     launch_fused<false, CfgFull, double, HALO, GAUGE>(plan, tiles, fg, FG_FULL, plan->dtab_full, io, prm, st);
     launch_fused<true, CfgWide, double, HALO, GAUGE>(plan, tiles, fg, FG_FACE, plan->dtab_wide, io, prm, st);
