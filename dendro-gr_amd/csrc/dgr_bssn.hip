@@ -2248,6 +2248,7 @@ struct dgr_plan {
         hipEvent_t a, b;
         double share;  // of the launch's time
         bool last;     // the launch's last entry: its events go back to the pool
+        bool counts;   // as a launch of its kind
     };
     std::vector<Timed> pending[DGR_TIMING_KINDS];
     double full_regular = 1.0;  // FP64 list: the 5-deep part's share of the points of the 6-7 deep tiles
@@ -2884,12 +2885,13 @@ int dgr_plan_kernel_times(dgr_plan *plan, double *ms, int64_t *launches) {
     HIP_OK(hipSetDevice(plan->device));
     for (int k = 0; k < DGR_TIMING_KINDS; k++) {
         ms[k] = 0.0;
-        launches[k] = (int64_t)plan->pending[k].size();
+        launches[k] = 0;
         for (auto &pr : plan->pending[k]) {
             HIP_OK(hipEventSynchronize(pr.b));
             float t = 0.f;
             HIP_OK(hipEventElapsedTime(&t, pr.a, pr.b));
             ms[k] += pr.share * t;
+            launches[k] += pr.counts;
             if (!pr.last) continue;
             plan->event_pool.push_back(pr.a);
             plan->event_pool.push_back(pr.b);
@@ -2943,9 +2945,10 @@ int load_ptrs(VarPtrs &vp, const double *const *src, const char *what) {
 
 // Runs `launch` on `st`, bracketed by timing events when the plan records them.
 // With `also` >= 0 (above `kind`) the launch counts there too, with the rest of
-// its time.
+// its time; without `counts` its time goes to another launch of `kind`.
 template <typename F>
-void timed(dgr_plan *plan, int kind, hipStream_t st, F launch, int also = -1, double share = 1.0) {
+void timed(dgr_plan *plan, int kind, hipStream_t st, F launch, int also = -1, double share = 1.0,
+           bool counts = true) {
     if (!plan->timing) {
         launch();
         return;
@@ -2955,8 +2958,8 @@ void timed(dgr_plan *plan, int kind, hipStream_t st, F launch, int also = -1, do
     launch();
     const bool rb = b && hipEventRecord(b, st) == hipSuccess;
     if (ra && rb) {
-        plan->pending[kind].push_back({a, b, share, also < 0});
-        if (also >= 0) plan->pending[also].push_back({a, b, 1.0 - share, true});
+        plan->pending[kind].push_back({a, b, share, also < 0, counts});
+        if (also >= 0) plan->pending[also].push_back({a, b, 1.0 - share, true, true});
     } else {  // an unrecorded pair would fail in dgr_plan_kernel_times: drop it
         if (a) plan->event_pool.push_back(a);
         if (b) plan->event_pool.push_back(b);
@@ -3056,12 +3059,13 @@ void launch_fused(dgr_plan *plan, const Tile *tiles, const int *fg, int group, i
     if (FP64) all[1] = all[0];
     void **args = all + FP64;
     // an FP64 launch on 6-7 deep tiles counts as the regular and the thin one it
-    // replaces, its time divided by their points
+    // replaces, its time divided by their points; as the regular one only if the
+    // stage has no launch of regular tiles, so that each kind counts once a stage
     const bool merged = FP64 && group == FG_FULL;
     timed(
         plan, 3 + (merged ? FG_WIDE : group), st,
         [&] { (void)hipLaunchKernel(fused_kernel<FACE, C, T, HALO, GAUGE>(), dim3(n), dim3(C::FT), args, 0, st); },
-        merged ? 3 + FG_THIN : -1, merged ? plan->full_regular : 1.0);
+        merged ? 3 + FG_THIN : -1, merged ? plan->full_regular : 1.0, !merged || fg[FG_WIDE + 1] == fg[FG_WIDE]);
 }
 
 // The FP64 launches of one tile list (groups as in fg).

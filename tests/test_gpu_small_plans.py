@@ -106,3 +106,22 @@ def test_one_launch_with_the_padding_refresh():
 
     a, b = both(t, steps)
     assert np.array_equal(a, b, equal_nan=True)
+
+
+def test_each_kind_counts_one_launch_a_stage():
+    """Kernel times of a plan with regular and 7-deep tiles: the 7-deep launch's
+    regular part adds its time to the regular launch's, not a launch."""
+    import torch
+    t = table(*CASES["wide+full"])
+    plan = dgr.Plan(t, W.total_padded(t))
+    plan.set_timing(True)
+    d = to_dev(host_state(t, seed=43))
+    out = torch.zeros_like(d)
+    log("launch counts by kind")
+    for _ in range(3):
+        plan.rhs(out, d, dgr.default_params())
+    torch.cuda.synchronize()
+    kt = plan.kernel_times()
+    plan.close()
+    assert kt["fused_wide"][1] == 3 and kt["fused_thin"][1] == 3, kt
+    assert kt["fused_wide"][0] > 0 and kt["fused_thin"][0] > 0
