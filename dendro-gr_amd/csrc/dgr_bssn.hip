@@ -1,6 +1,7 @@
 // MI355X (gfx950) BSSN right-hand side over a batch of padded octree blocks.
 //
-// Work decomposition
+// Work decomposition of the split path (DGR_KERNEL=split); by default one kernel
+// does a whole stage, k_stream (stream_fp64.h) in FP64 and k_fused in FP32
 //   * every block's interior is cut into tiles of at most 7x7x7 points
 //     (a 13^3 block is one tile, a 55^3 block 343 tiles);
 //   * tiles are grouped into chunks of whole blocks whose derivative
@@ -649,11 +650,13 @@ enum { FG_WIDE = 0, FG_THIN = 1, FG_FACE = 2, FG_FULL = 3, NFGROUP = 4 };
 enum { SCH_WT = 0, SCH_W = 1, SCH_FULL = 2, NSCHEME = 3 };
 
 // Where a stage reads its state and writes its results. Stage buffers hold
-// interior points only, indexed by DBlock::q0 + (i-3) + mx*((j-3) + my*(k-3));
+// interior points only, indexed by DBlock::q0 + (i-3) + mx*((j-3) + my*(k-3))
+// (the FP64 stage kernels': in their lanes' order, StreamIO);
 // padding always comes from the caller's state `u`.
 // Buffers of one fused launch. An RK4 step alternates two padded states: the
 // caller's u and the plan's work state W, whose padding holds a copy of u's
-// (k_pad_copy, once per dgr_rk4_step / dgr_rk4_steps call). Stage 0 reads u
+// (k_block_copy, or k_pad_copy where stages refresh the linked padding; once per
+// dgr_rk4_step / dgr_rk4_steps call). Stage 0 reads u
 // and writes the next stage state into W's interior; stage 1 reads W and
 // writes u's interior; stage 2 reads u and writes W; stage 3 reads W and
 // writes the result into u. A stage therefore reads its whole region from
