@@ -142,8 +142,9 @@ class Workload:
 KERNEL_SOURCES = ("dendro-gr_amd/csrc/dgr_bssn.hip", "dendro-gr_amd/csrc/stencils.h",
                   "dendro-gr_amd/csrc/bssn_rhs_phased.h", "dendro-gr_amd/csrc/bssn_rhs_generated.h",
                   "dendro-gr_amd/csrc/bssn_ham_generated.h", "dendro-gr_amd/csrc/bssn_cons_phased.h",
-                  "dendro-gr_amd/csrc/bssn_rhs_stream.h", "dendro-gr_amd/csrc/stream_fp64.h", "dendro-gr_amd/csrc/bssn_rhs_gauge_generated.h",
-                  "dendro-gr_amd/build.py")
+                  "dendro-gr_amd/csrc/bssn_rhs_stream.h", "dendro-gr_amd/csrc/stream_fp64.h",
+                  "dendro-gr_amd/csrc/stream_tile.h", "dendro-gr_amd/csrc/bssn_rhs_gauge_generated.h",
+                  "include/dgr_bssn.h", "dendro-gr_amd/build.py")
 
 
 def source_sha():
