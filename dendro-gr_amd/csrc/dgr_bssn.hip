@@ -1267,6 +1267,28 @@ struct ConsFusedOut {
     __device__ __forceinline__ void put(double x) { v[I] = x; }
 };
 
+// The tile of one k_cons_fused workgroup: its list is the FP64 stage kernels',
+// whose 6-7 deep tiles this kernel (one workgroup of 256 threads a CU) takes in
+// two launches, C = CfgWide the first 5 planes and C = CfgThin the rest, with the lane
+// tables behind the deep shape's own (deep_lane_tables). A tile list of its own
+// cost the plan of 30 M points of uneven octree 4 of 14 ms to create, and a plan is
+// made again at every regrid; the calls take the same time either way (5 M points of
+// refined octree with the norm 2.06 ms).
+template <class C>
+__device__ __forceinline__ Tile cons_tile(Tile t) {
+    constexpr bool REST = C::FT == CfgThin::FT;
+    if (REST || t.e[2] > CfgWide::FZ) {
+        t.lanetab += 2 * CfgFull::FT + (REST ? 2 * CfgWide::FT : 0);
+        if (REST) {
+            t.o[2] += CfgWide::FZ;
+            t.e[2] -= CfgWide::FZ;
+        } else {
+            t.e[2] = CfgWide::FZ;
+        }
+    }
+    return t;
+}
+
 template <bool FACE, class C>
 __global__ __launch_bounds__(C::FT, 1) void k_cons_fused(const StageIO io, ConsPtrs o,
                                                         const DBlock *__restrict__ blocks,
@@ -1278,7 +1300,7 @@ __global__ __launch_bounds__(C::FT, 1) void k_cons_fused(const StageIO io, ConsP
     __shared__ double s_tile[(DEEP ? 3 : 2) * C::NREG];
     __shared__ double s_dx[(DEEP ? 2 : 1) * C::NSDX];
     __shared__ double s_dy[(DEEP ? 2 : 1) * C::NSDY];
-    const Tile tl = tiles[blockIdx.x];
+    const Tile tl = cons_tile<C>(tiles[blockIdx.x]);
     const DBlock B = blocks[tl.block];
     Ctx ctx(io);
     ctx.K = bconst + 3 * (size_t)tl.block;
@@ -2198,11 +2220,11 @@ struct dgr_plan {
     double *d_stage = nullptr;  // split path RK4: 2 * 24 * szpdof (stage state, accumulator)
     bool fused = true;          // k_fused (default) or the split k_derivs/k_rhs path (DGR_KERNEL=split)
     int precision = DGR_PRECISION_FP64;  // arithmetic of the fused kernel
-    // tile lists (LIST_FP64, LIST_MIXED, LIST_CONS), XCD-grouped, group k in
+    // tile lists per precision (0 FP64, 1 mixed), XCD-grouped, group k in
     // [fgroup[p][k], fgroup[p][k+1]), each interior block tiled by the scheme
     // tiling[p] holds for its size (else the default of tiling_of)
-    Tile *d_ftiles[3] = {};
-    int fgroup[3][NFGROUP + 1] = {};
+    Tile *d_ftiles[2] = {};
+    int fgroup[2][NFGROUP + 1] = {};
     std::map<std::array<int, 3>, int> tiling[2];
     std::vector<DBlock> hblocks;                  // host copy of the block table
     std::map<std::array<int, 4>, int> lane_off;   // lane table offset per (ex, ey, ez, threads)
@@ -2311,6 +2333,14 @@ void lane_table(int ex, int ey, int ez, int ft, std::vector<uint16_t> &out) {
     for (int l = 0; l < ft; l++) out.push_back(rank[out[first + l] & (LANE_SHADOW - 1)]);
 }
 
+// Behind the lane table of a 6-7 deep shape: those of its first 5 planes and of
+// the rest, in the shapes k_cons_fused takes them in (cons_tile).
+void deep_lane_tables(int ex, int ey, int ez, std::vector<uint16_t> &out) {
+    if (ez <= CfgWide::FZ) return;
+    lane_table(ex, ey, CfgWide::FZ, CfgWide::FT, out);
+    lane_table(ex, ey, ez - CfgWide::FZ, CfgThin::FT, out);
+}
+
 // Slot table of a tile configuration: slot (it, tid) -> the position
 // w = i0 + 13 j + 169 k it evaluates and writes, first D_x for DXIT passes,
 // then D_y for DYIT passes, grouped like lane_table; unused slots get w = 7
@@ -2407,13 +2437,9 @@ int thread_count(int group) {
     return group == FG_THIN ? CfgThin::FT : group == FG_FULL ? CfgFull::FT : CfgWide::FT;
 }
 
-// The tile lists of a plan: the FP64 stage kernels', the mixed-precision ones'
-// and the constraints'.
-enum { LIST_FP64 = 0, LIST_MIXED = 1, LIST_CONS = 2, NLIST = 3 };
-
 // The tiles of one group by slot (block), slots filled in increasing order, in one
-// array (with a vector a slot and three table look-ups a tile, the plan of 30 M
-// points of uneven octree took 22.8 ms to create, now 17.6).
+// array (a vector a slot and three table look-ups a tile made the plan of 30 M
+// points of uneven octree 5 ms slower to create; now 9.7 ms).
 struct TileGroup {
     std::vector<Tile> tiles;
     std::vector<uint32_t> begin;  // first tile of each slot so far
@@ -2427,8 +2453,9 @@ struct TileGroup {
     const Tile &at(size_t slot, size_t k) const { return tiles[begin[slot] + k]; }
 };
 
-// Appends list `p`'s tiles of block b under scheme `sch` to per[group], slot `slot`.
-// In the FP64 list a remainder of 1-2 points joins the 5 before it in a tile of
+// Appends the tiles of block b under scheme `sch` in precision p (0 FP64, 1
+// mixed) to per[group], slot `slot`.
+// In FP64 a remainder of 1-2 points joins the 5 before it in a tile of
 // the 7-deep shape: a thin tile of its own stages and differentiates 6 planes
 // of halo for its 2 (on 13^3 blocks, 4096 of them, the two launches of a stage
 // fetched 3.3 GB where one fetches 2.4). Blocks
@@ -2445,7 +2472,7 @@ void block_tiles(const DBlock &d, uint32_t b, int p, int sch, TileGroup *per, si
         split_axis_max(d.n[2] - 6, CfgFull::FZ, pz);
     } else {
         for (int o = PW, m = d.n[2] - 6; m > 0;) {
-            const int e = std::min(m, p == LIST_FP64 && m <= CfgFull::FZ ? CfgFull::FZ : CfgWide::FZ);
+            const int e = std::min(m, p == 0 && m <= CfgFull::FZ ? CfgFull::FZ : CfgWide::FZ);
             pz.push_back({o, e});
             o += e;
             m -= e;
@@ -2474,6 +2501,9 @@ void block_tiles(const DBlock &d, uint32_t b, int p, int sch, TileGroup *per, si
 // round-robin over the 8 XCDs the tiles of one block share an XCD and its L2
 // for their overlapping halos.
 void group_tiles(const TileGroup *per, std::vector<Tile> &out, int *fgroup) {
+    size_t n = 0;
+    for (int g = 0; g < NFGROUP; g++) n += per[g].tiles.size();
+    out.reserve(n);
     for (int g = 0; g < NFGROUP; g++) {
         fgroup[g] = (int)out.size();
         std::vector<size_t> bl;
@@ -2544,13 +2574,13 @@ hipError_t build_ftiles(dgr_plan *plan, int p) {
     TileGroup per[NFGROUP];
     for (size_t b = 0; b < nb; b++) {
         const DBlock &d = plan->hblocks[b];
-        block_tiles(d, (uint32_t)b, p, d.bflag ? SCH_WT : tiling_of(plan, p == LIST_MIXED, d), per, b);
+        block_tiles(d, (uint32_t)b, p, d.bflag ? SCH_WT : tiling_of(plan, p, d), per, b);
     }
     std::vector<Tile> tiles;
     int fg[NFGROUP + 1];
     group_tiles(per, tiles, fg);
     if (!assign_lane_tables(plan, tiles, fg)) return hipErrorInvalidValue;
-    if (p == LIST_FP64) {
+    if (p == 0) {
         double regular = 0.0, all = 0.0;
         for (int i = fg[FG_FULL]; i < fg[FG_FULL + 1]; i++) {
             const int *e = tiles[i].e;
@@ -2720,18 +2750,6 @@ int dgr_plan_create(int device, const dgr_block *blocks, uint32_t nblocks, uint6
     tabs_ok = dtable<CfgThin>(tabs) && tabs_ok;
     plan->dtab_full = (int)tabs.size();
     tabs_ok = dtable<CfgFull>(tabs) && tabs_ok;
-    // (blocks are at least 13 wide, so near-equal parts are 4 to 7 points)
-    for (int ex = 4; ex <= TMAX; ex++)
-        for (int halo = 0; halo < 2; halo++) {
-            plan->stage_off[{ex, SWide::FT, halo}] = (int)tabs.size();
-            tabs_ok = stage_table<SWide>(halo, ex, tabs) && tabs_ok;
-            plan->stage_off[{ex, SFull::FT, halo}] = (int)tabs.size();
-            tabs_ok = stage_table<SFull>(halo, ex, tabs) && tabs_ok;
-        }
-    if (!tabs_ok) {
-        dgr_plan_destroy(plan);
-        return fail(DGR_E_INVALID, "internal error: D_x / D_y slot table does not match its configuration");
-    }
     {
         std::map<std::array<int, 4>, bool> seen;
         for (uint32_t b = 0; b < nblocks; b++) {
@@ -2740,16 +2758,28 @@ int dgr_plan_create(int device, const dgr_block *blocks, uint32_t nblocks, uint6
                 continue;
             for (int sch = 0; sch < (d.bflag ? 1 : NSCHEME); sch++) {
                 TileGroup per[NFGROUP];
-                for (int p = 0; p < NLIST; p++) block_tiles(d, b, p, sch, per, 0);
+                for (int p = 0; p < 2; p++) block_tiles(d, b, p, sch, per, 0);
                 for (int g = 0; g < NFGROUP; g++)
                     for (const Tile &t : per[g].tiles) {
                         const std::array<int, 4> key{t.e[0], t.e[1], t.e[2], thread_count(g)};
                         if (plan->lane_off.count(key)) continue;
                         plan->lane_off[key] = (int)tabs.size();
                         lane_table(t.e[0], t.e[1], t.e[2], thread_count(g), tabs);
+                        if (g == FG_FULL) deep_lane_tables(t.e[0], t.e[1], t.e[2], tabs);
+                        for (int halo = 0; halo < 2 && g != FG_THIN; halo++) {
+                            const std::array<int, 3> stage{t.e[0], thread_count(g), halo};
+                            if (plan->stage_off.count(stage)) continue;
+                            plan->stage_off[stage] = (int)tabs.size();
+                            tabs_ok = (g == FG_FULL ? stage_table<SFull>(halo, t.e[0], tabs)
+                                                    : stage_table<SWide>(halo, t.e[0], tabs)) && tabs_ok;
+                        }
                     }
             }
         }
+    }
+    if (!tabs_ok) {
+        dgr_plan_destroy(plan);
+        return fail(DGR_E_INVALID, "internal error: D_x / D_y slot table does not match its configuration");
     }
     std::vector<dgr::AxisConsts> bconst(3 * (size_t)nblocks);
     for (uint32_t b = 0; b < nblocks; b++)
@@ -2777,7 +2807,7 @@ int dgr_plan_create(int device, const dgr_block *blocks, uint32_t nblocks, uint6
     if (e == hipSuccess && !wg_tile.empty()) e = hipMemcpy(plan->d_wg_tile, wg_tile.data(), sizeof(int) * wg_tile.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess && !face_tiles.empty())
         e = hipMemcpy(plan->d_face_tiles, face_tiles.data(), sizeof(int) * face_tiles.size(), hipMemcpyHostToDevice);
-    for (int p = 0; p < NLIST && e == hipSuccess; p++) e = build_ftiles(plan, p);
+    for (int p = 0; p < 2 && e == hipSuccess; p++) e = build_ftiles(plan, p);
     if (e == hipSuccess) e = hipMemset(plan->d_err, 0, sizeof(int));
     if (e != hipSuccess) {
         dgr_plan_destroy(plan);
@@ -2807,7 +2837,6 @@ int dgr_plan_destroy(dgr_plan *plan) {
     (void)hipFree(plan->d_stage);
     (void)hipFree(plan->d_ftiles[0]);
     (void)hipFree(plan->d_ftiles[1]);
-    (void)hipFree(plan->d_ftiles[2]);
     (void)hipFree(plan->d_bconst);
     (void)hipFree(plan->d_tabs);
     (void)hipFree(plan->d_istage);
@@ -3227,7 +3256,6 @@ int dgr_plan_autotune(dgr_plan *plan, double *const *d_rhs, const double *const 
             plan->tiling[p][kv.first] = best;
         }
         HIP_OK(build_ftiles(plan, p));
-        if (!p) HIP_OK(build_ftiles(plan, LIST_CONS));
         if (plan->rk4_exec) {  // the captured step used the previous tile list
             HIP_OK(hipGraphExecDestroy(plan->rk4_exec));
             plan->rk4_exec = nullptr;
@@ -3253,7 +3281,6 @@ int dgr_plan_set_tiling(dgr_plan *plan, int precision, uint32_t nx, uint32_t ny,
     plan->tiling[p][{(int)nx, (int)ny, (int)nz}] = scheme;
     HIP_OK(hipSetDevice(plan->device));
     HIP_OK(build_ftiles(plan, p));
-    if (!p) HIP_OK(build_ftiles(plan, LIST_CONS));
     if (plan->rk4_exec) {  // the captured step used the previous tile list
         HIP_OK(hipGraphExecDestroy(plan->rk4_exec));
         plan->rk4_exec = nullptr;
@@ -4143,20 +4170,17 @@ int dgr_constraints(dgr_plan *plan, double *d_ham, double *const *d_mom, double 
         StageIO io{};
         io.src = u;
         io.stage = -1;
-        const Tile *tiles = plan->d_ftiles[LIST_CONS];
-        const int *fg = plan->fgroup[LIST_CONS];
-        int n = fg[FG_WIDE + 1] - fg[FG_WIDE];
-        if (n)
-            hipLaunchKernelGGL((k_cons_fused<false, CfgWide>), dim3(n), dim3(CfgWide::FT), 0, st, io, o,
-                               plan->d_blocks, plan->d_bconst, tiles + fg[FG_WIDE], plan->d_tabs, plan->dtab_wide);
-        n = fg[FG_THIN + 1] - fg[FG_THIN];
-        if (n)
-            hipLaunchKernelGGL((k_cons_fused<false, CfgThin>), dim3(n), dim3(CfgThin::FT), 0, st, io, o,
-                               plan->d_blocks, plan->d_bconst, tiles + fg[FG_THIN], plan->d_tabs, plan->dtab_thin);
-        n = fg[FG_FACE + 1] - fg[FG_FACE];
-        if (n)
-            hipLaunchKernelGGL((k_cons_fused<true, CfgWide>), dim3(n), dim3(CfgWide::FT), 0, st, io, o,
-                               plan->d_blocks, plan->d_bconst, tiles + fg[FG_FACE], plan->d_tabs, plan->dtab_wide);
+        const int *fg = plan->fgroup[0];
+        auto launch = [&](auto kernel, int group, int threads, int dtab) {
+            const int n = fg[group + 1] - fg[group];
+            if (n)
+                hipLaunchKernelGGL(kernel, dim3(n), dim3(threads), 0, st, io, o, plan->d_blocks, plan->d_bconst,
+                                   plan->d_ftiles[0] + fg[group], plan->d_tabs, dtab);
+        };
+        launch(k_cons_fused<false, CfgWide>, FG_WIDE, CfgWide::FT, plan->dtab_wide);
+        launch(k_cons_fused<false, CfgWide>, FG_FULL, CfgWide::FT, plan->dtab_wide);
+        launch(k_cons_fused<false, CfgThin>, FG_FULL, CfgThin::FT, plan->dtab_thin);
+        launch(k_cons_fused<true, CfgWide>, FG_FACE, CfgWide::FT, plan->dtab_wide);
         HIP_OK(hipGetLastError());
         return DGR_OK;
     }
