@@ -3100,16 +3100,37 @@ void launch_fused(dgr_plan *plan, const Tile *tiles, const int *fg, int group, i
         merged ? 3 + FG_THIN : -1, merged ? plan->full_regular : 1.0, !merged || fg[FG_WIDE + 1] == fg[FG_WIDE]);
 }
 
-// The FP64 launches of one tile list (groups as in fg).
+// Whether FP64 stages over these tile groups are one launch: at most a tile for
+// each CU, of more than one kind. Of one kind, or with more tiles, where two of
+// the smaller workgroups share a CU: a launch a kind.
+bool one_launch(const int *fg) {
+    const int wide = fg[FG_FACE] - fg[FG_WIDE], face = fg[FG_FULL] - fg[FG_FACE], full = fg[NFGROUP] - fg[FG_FULL];
+    return (wide > 0) + (face > 0) + (full > 0) > 1 && wide + face + full <= SMALL_TILES;
+}
+
+// The same for the plan's list with its unflagged blocks of size n tiled by sch.
+bool one_launch_tiled(const dgr_plan *plan, const std::array<int, 3> &n, int sch) {
+    int fg[NFGROUP + 1] = {};
+    if (plan->hblocks.size() > SMALL_TILES) return false;  // at least a tile a block
+    for (const DBlock &d : plan->hblocks) {
+        TileGroup per[NFGROUP];
+        const bool tuned = d.n[0] == n[0] && d.n[1] == n[1] && d.n[2] == n[2];
+        block_tiles(d, 0, 0, d.bflag ? SCH_WT : tuned ? sch : tiling_of(plan, 0, d), per, 0);
+        for (int g = 0, before = 0; g < NFGROUP; g++) {
+            before += (int)per[g].tiles.size();
+            fg[g + 1] += before;
+        }
+        if (fg[NFGROUP] > SMALL_TILES) return false;
+    }
+    return one_launch(fg);
+}
+
+// The FP64 launches of one tile list (groups as in fg): in one, or kind by kind.
 template <bool HALO, bool GAUGE>
 void launch_stream(dgr_plan *plan, const Tile *tiles, const int *fg, const StageIO &io, const RhsParams &prm,
-                   hipStream_t st) {
-    // At most a tile for each CU, of more than one kind: one launch (with timing
-    // on a launch a kind, so that each has its own time). Of one kind, or with
-    // more tiles, where two of the smaller workgroups share a CU: a launch a kind.
-    const int nface = fg[FG_FULL] - fg[FG_FACE], nfull = fg[NFGROUP] - fg[FG_FULL], n = fg[NFGROUP] - fg[FG_WIDE];
-    const int kinds = (n > nface + nfull) + (nface > 0) + (nfull > 0);
-    if (kinds > 1 && n <= SMALL_TILES && !plan->timing) {
+                   hipStream_t st, bool one) {
+    if (one) {
+        const int nface = fg[FG_FULL] - fg[FG_FACE], nfull = fg[NFGROUP] - fg[FG_FULL], n = fg[NFGROUP] - fg[FG_WIDE];
         static const void *const *tab = [] {
             static const void *k[4];
             dgr_internal_small_kernels(k);
@@ -3129,13 +3150,13 @@ void launch_stream(dgr_plan *plan, const Tile *tiles, const int *fg, const Stage
 
 template <typename T>
 void launch_fused_all(dgr_plan *plan, const Tile *tiles, const int *fg, const StageIO &io, const RhsParams &prm,
-                      hipStream_t st) {
+                      hipStream_t st, bool one = false) {
     if constexpr (sizeof(T) == sizeof(double)) {
         const bool gauge = gauge_variant(prm);  // the reference's other builds (FP64 only)
-        if (io.nbo && gauge) launch_stream<true, true>(plan, tiles, fg, io, prm, st);
-        else if (io.nbo) launch_stream<true, false>(plan, tiles, fg, io, prm, st);
-        else if (gauge) launch_stream<false, true>(plan, tiles, fg, io, prm, st);
-        else launch_stream<false, false>(plan, tiles, fg, io, prm, st);
+        if (io.nbo && gauge) launch_stream<true, true>(plan, tiles, fg, io, prm, st, one);
+        else if (io.nbo) launch_stream<true, false>(plan, tiles, fg, io, prm, st, one);
+        else if (gauge) launch_stream<false, true>(plan, tiles, fg, io, prm, st, one);
+        else launch_stream<false, false>(plan, tiles, fg, io, prm, st, one);
     } else if (io.nbo) {  // the padding refresh inside the stage kernel
         launch_fused<false, CfgOf<float>::Wide, T, true>(plan, tiles, fg, FG_WIDE, plan->dtab_wide, io, prm, st);
         launch_fused<false, CfgOf<float>::Thin, T, true>(plan, tiles, fg, FG_THIN, plan->dtab_thin, io, prm, st);
@@ -3156,7 +3177,9 @@ int run_fused(dgr_plan *plan, const StageIO &io, const RhsParams &prm, hipStream
     if (plan->precision == DGR_PRECISION_MIXED)
         launch_fused_all<float>(plan, plan->d_ftiles[1], plan->fgroup[1], io, prm, st);
     else
-        launch_fused_all<double>(plan, plan->d_ftiles[0], plan->fgroup[0], io, prm, st);
+        // (with timing on a launch a kind, so that each has its own time)
+        launch_fused_all<double>(plan, plan->d_ftiles[0], plan->fgroup[0], io, prm, st,
+                                 one_launch(plan->fgroup[0]) && !plan->timing);
     HIP_OK(hipGetLastError());
     return DGR_OK;
 }
@@ -3236,11 +3259,12 @@ int dgr_plan_autotune(dgr_plan *plan, double *const *d_rhs, const double *const 
                     cap = tiles.size();
                 }
                 HIP_OK(hipMemcpy(d_t, tiles.data(), sizeof(Tile) * tiles.size(), hipMemcpyHostToDevice));
+                const bool one = p == 0 && one_launch_tiled(plan, kv.first, sch);  // as the plan would run it
                 float ms = 0.f;
                 for (int rep = 0; rep < 4; rep++) {  // a warm-up, then the best of three
                     HIP_OK(hipEventRecord(e0, st));
                     if (p) launch_fused_all<float>(plan, d_t, fg, io, prm, st);
-                    else launch_fused_all<double>(plan, d_t, fg, io, prm, st);
+                    else launch_fused_all<double>(plan, d_t, fg, io, prm, st, one);
                     HIP_OK(hipGetLastError());
                     HIP_OK(hipEventRecord(e1, st));
                     HIP_OK(hipEventSynchronize(e1));
