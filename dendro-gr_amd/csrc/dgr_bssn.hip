@@ -579,13 +579,10 @@ constexpr int DXS_Y = FRX, DXS_Z = FRXY;
 constexpr int DYS_Y = FRX, DYS_Z = FRXY;
 constexpr int LANE_SHADOW = 0x8000;  // lane table: the lane repeats a point and stores nothing
 
-// Tile shape of a k_fused launch: FT threads (one point each) and tiles of at
-// most 7 x 7 x FZ points. The regular shape is 256 threads / z <= 5 (one
-// workgroup per CU: it takes 143 KB of LDS); the thin shape, 128 threads /
-// z <= 2, takes the 2-point z remainder of a block (a 13^3 block's interior
-// is 7x7x5 + 7x7x2) in half the threads and ~80 KB, so two share a CU.
-// PD variables are fetched ahead of the one being differentiated: with a
-// single wave per SIMD, the loads in flight are what keeps HBM busy.
+// Tile shape of a launch: FT threads (one point each) and tiles of at most
+// 7 x 7 x FZ points: 256 threads / z <= 5, 128 / z <= 2 (a 7-point interior as
+// 5 + 2 takes 384 threads) and 384 / z <= 7. PD variables are fetched ahead of
+// the one being differentiated.
 template <int FT_, int FZ_, int PD_>
 struct FCfg {
     static constexpr int FT = FT_;
@@ -601,44 +598,36 @@ struct FCfg {
     static constexpr int DYIT = (NDY + FT - 1) / FT;
     static constexpr int NSDX = TMAX + FRX * (RMAX - 1) + FRXY * (FZ + 2 * PW - 1);  // D_x array
     static constexpr int NSDY = TMAX + FRX * (TMAX - 1) + FRXY * (FZ + 2 * PW - 1);  // D_y array
-    // LDS (FP64 kernel): two region buffers, D_x / D_y, KO terms
-    static constexpr size_t LDS = sizeof(double) * (2 * NREG + NSDX + NSDY + NV * FT);
 };
+// The constraint kernel, FP64 (their fields fill the registers, so a SIMD runs one
+// wave: the loads in flight are what keeps HBM busy). Regular tiles have three region
+// buffers and two D_x / D_y sets (one barrier a phase), thin ones two and one.
 using CfgWide = FCfg<256, 5, 3>;
 using CfgThin = FCfg<128, 2, 2>;
-// FP32 kernel on interior blocks: a whole 7 x 7 x 7 column per workgroup
-// (384 threads, ~98 KB of LDS, one workgroup per CU). Its registers allow two
-// waves per SIMD, so six waves fit where the FP64 kernel fits four: a 13^3
-// block's interior is one tile, and the staging and D_x / D_y work of the
-// z halo is shared by 7 planes instead of 5 + 2.
-using CfgFull = FCfg<384, 7, 1>;
-// The FP32 kernels fit two waves per SIMD in 256 registers only with one
-// variable in flight.
-template <typename T>
-struct CfgOf {
-    using Wide = CfgWide;
-    using Thin = CfgThin;
-};
-template <>
-struct CfgOf<float> {
-    using Wide = FCfg<256, 5, 1>;
-    using Thin = FCfg<128, 2, 1>;
-};
-static_assert(7 * 7 * CfgWide::FZ <= CfgWide::FT && 7 * 7 * CfgThin::FZ <= CfgThin::FT, "one point per thread");
-static_assert(2 * CfgThin::LDS <= 160 * 1024, "two thin FP64 workgroups per CU");
-// FP32 regular tiles: one FP64 and one FP32 region buffer, FP64-sized D_x /
-// D_y arrays (alpha and chi are differentiated in FP64), FP32 KO terms
-static_assert(2 * (sizeof(double) * (CfgWide::NREG + (CfgWide::NREG + 1) / 2 + CfgWide::NSDX + CfgWide::NSDY) +
-                   sizeof(float) * NV * CfgWide::FT) <= 160 * 1024,
+static_assert(sizeof(double) * (3 * CfgWide::NREG + 2 * (CfgWide::NSDX + CfgWide::NSDY)) <= 160 * 1024,
+              "one regular workgroup per CU");
+static_assert(2 * sizeof(double) * (2 * CfgThin::NREG + CfgThin::NSDX + CfgThin::NSDY) <= 160 * 1024,
+              "two thin workgroups per CU");
+// The FP32 stage kernels, at two waves a SIMD in 256 registers, which leaves room
+// for one variable in flight. Regular tiles: one FP64 and one FP32 region
+// buffer, FP64-sized D_x / D_y arrays (alpha and chi are differentiated in
+// FP64), FP32 KO terms.
+using F32Wide = FCfg<256, 5, 1>;
+using F32Thin = FCfg<128, 2, 1>;
+static_assert(2 * (sizeof(double) * (F32Wide::NREG + (F32Wide::NREG + 1) / 2 + F32Wide::NSDX + F32Wide::NSDY) +
+                   sizeof(float) * NV * F32Wide::FT) <= 160 * 1024,
               "two FP32 workgroups per CU");
-static_assert(7 * 7 * CfgFull::FZ <= CfgFull::FT, "one point per thread");
-// three FP64-sized region buffers and two D_x / D_y buffers (one barrier per phase)
+// A whole 7 x 7 x 7 column per workgroup (a 13^3 block's interior is one tile,
+// and the staging and D_x / D_y work of the z halo is shared by 7 planes instead
+// of 5 + 2), six waves and one workgroup a CU: FP32 with three FP64-sized region
+// buffers and two D_x / D_y sets (one barrier a phase); in FP64 SCfg.
+using CfgFull = FCfg<384, 7, 1>;
 static_assert(sizeof(double) * (3 * CfgFull::NREG + 2 * (CfgFull::NSDX + CfgFull::NSDY)) +
                       sizeof(float) * NV * CfgFull::FT <= 160 * 1024,
               "one FP32 7x7x7 workgroup per CU");
-static_assert(sizeof(double) * (3 * CfgWide::NREG + 2 * (CfgWide::NSDX + CfgWide::NSDY) + NV * CfgWide::FT) <=
-                  160 * 1024,
-              "one FP64 regular workgroup per CU");
+static_assert(7 * 7 * CfgWide::FZ <= CfgWide::FT && 7 * 7 * CfgThin::FZ <= CfgThin::FT &&
+                  7 * 7 * CfgFull::FZ <= CfgFull::FT,
+              "one point per thread");
 // tile groups of the fused path, one launch each (FULL: FP32 only)
 enum { FG_WIDE = 0, FG_THIN = 1, FG_FACE = 2, FG_FULL = 3, NFGROUP = 4 };
 // Tilings of a block without flagged faces, chosen per block size and
@@ -803,7 +792,7 @@ struct FusedCtx {
     // buffer K&1 by phase K-2, both before barrier K-1, which every wave has
     // passed when it writes them in phase K. Other kernels keep two region
     // buffers and two barriers in phases with mixed derivatives.
-    static constexpr bool DEEP = sizeof(T) == sizeof(double) ? C::FT == CfgWide::FT : C::FT == CfgFull::FT;
+    static constexpr bool DEEP = C::FT == (sizeof(T) == sizeof(double) ? CfgWide::FT : CfgFull::FT);
     template <int K>
     static constexpr int rbuf() { return DEEP ? K % 3 : K & 1; }
 
@@ -987,16 +976,16 @@ struct FusedCtx {
 // The equations' outputs: on a flagged face the boundary value (already
 // holding its KO term), elsewhere equations + KO term, kept in LDS until the
 // epilogue.
-template <bool FACE, class C, typename T, bool HALO, class P = RhsPhases>
+template <bool FACE, class C, bool HALO>
 struct FusedOut {
     static constexpr int FT = C::FT;
-    const FusedCtx<FACE, C, T, P, HALO> &ctx;
-    __device__ explicit FusedOut(const FusedCtx<FACE, C, T, P, HALO> &c) : ctx(c) {}
+    const FusedCtx<FACE, C, float, RhsPhases, HALO> &ctx;
+    __device__ explicit FusedOut(const FusedCtx<FACE, C, float, RhsPhases, HALO> &c) : ctx(c) {}
     template <int V>
-    __device__ __forceinline__ void put(T val) {
+    __device__ __forceinline__ void put(float val) {
 #pragma clang fp contract(off)
-        T *s = ctx.s_ko + V * FT + ctx.tid;
-        const T kb = *s;
+        float *s = ctx.s_ko + V * FT + ctx.tid;
+        const float kb = *s;
         *s = (FACE && ctx.face) ? kb : val + kb;
     }
 };
@@ -1005,11 +994,11 @@ struct FusedOut {
 // loads of all 24 variables issued before any store. Stage s (U = {0, 1/2,
 // 1/2, 1}, C = {1/6, 1/3, 1/3, 1/6}): acc = (s ? acc : u0) + C[s] dt k;
 // next = u0 + U[s+1] dt k (s < 3) or the final state acc (s = 3).
-// The RK arithmetic is FP64 in both precisions; the mixed path's FP32
-// right-hand side is widened first and its u0 read back in FP64.
-template <class C, typename T>
-__device__ __forceinline__ void fused_epilogue(const StageIO &io, const T *s_ko, const T *f, int tid,
-                                               uint64_t idx, int64_t q, double chi_floor) {
+// The RK arithmetic is FP64: the FP32 right-hand side is widened first and u0
+// read back in FP64.
+template <class C>
+__device__ __forceinline__ void fused_epilogue(const StageIO &io, const float *s_ko, int tid, uint64_t idx, int64_t q,
+                                               double chi_floor) {
 #pragma clang fp contract(off)
     constexpr int FT = C::FT;
     const int s = io.stage;
@@ -1019,10 +1008,7 @@ __device__ __forceinline__ void fused_epilogue(const StageIO &io, const T *s_ko,
         return;
     }
     double u0[NV], a0[NV], v14[14];
-    if (s == 0 && sizeof(T) == sizeof(double)) {
-#pragma unroll
-        for (int v = 0; v < NV; v++) u0[v] = a0[v] = double(f[v]);
-    } else if (s == 0) {
+    if (s == 0) {
 #pragma unroll
         for (int v = 0; v < NV; v++) u0[v] = a0[v] = io.src.p[v][idx];
     } else {
@@ -1178,11 +1164,12 @@ __device__ __forceinline__ void tile_setup(FusedCtx<FACE, C, T, P, HALO> &ctx, c
     active_out = active;
 }
 
-template <bool FACE, class C, typename T, bool HALO = false, class P = RhsPhases>
+template <bool FACE, class C, bool HALO>
 __device__ __forceinline__ void fused_tile(const StageIO &io, const RhsParams &prm, const Tile &tl, const DBlock &B,
                                            const dgr::AxisConsts *K, const uint16_t *__restrict__ tabs,
-                                           int dtab, double *s_tile, double *s_dx, double *s_dy, T *s_ko) {
-    FusedCtx<FACE, C, T, P, HALO> ctx(io);
+                                           int dtab, double *s_tile, double *s_dx, double *s_dy, float *s_ko) {
+    using T = float;
+    FusedCtx<FACE, C, T, RhsPhases, HALO> ctx(io);
     ctx.K = K;
     ctx.load_consts();
     ctx.s_tile = s_tile;
@@ -1211,39 +1198,35 @@ __device__ __forceinline__ void fused_tile(const StageIO &io, const RhsParams &p
     const T lam[4] = {T(prm.lam[0]), T(prm.lam[1]), T(prm.lam[2]), T(prm.lam[3])};
     const T lamf[2] = {T(prm.lamf[0]), T(prm.lamf[1])};
     ctx.template fetch<0>();
-    if constexpr (C::PD > 1) ctx.template fetch<1>();
-    if constexpr (C::PD > 2) ctx.template fetch<2>();
-    static_assert(C::PD <= 3, "prefetch distance");
+    static_assert(C::PD == 1, "prefetch distance");
     ctx.begin();
-    FusedOut<FACE, C, T, HALO, P> out(ctx);
+    FusedOut<FACE, C, HALO> out(ctx);
     dgr::bssn_rhs_phased<T>(ctx, ctx.eta_v, lam, lamf, out);
-    if (active) fused_epilogue<C, T>(io, s_ko, ctx.f, ctx.tid, idx, q, prm.chi_floor);
+    if (active) fused_epilogue<C>(io, s_ko, ctx.tid, idx, q, prm.chi_floor);
 }
 
-// One launch per tile kind: FACE = false over the tiles of blocks without
-// flagged faces, FACE = true over the others; C the tile shape; T the
-// arithmetic type (FP32 asks for two waves per SIMD: its registers allow it).
+// The FP32 stage kernel. One launch per tile kind: FACE = false over the tiles of
+// blocks without flagged faces, FACE = true over the others; C the tile shape.
 #ifndef DGR_FP32_WAVES
-#define DGR_FP32_WAVES 2  // waves per SIMD the FP32 kernels are built for
+#define DGR_FP32_WAVES 2  // waves per SIMD it is built for
 #endif
 
-template <bool FACE, class C, typename T, bool HALO = false>
-__global__ __launch_bounds__(C::FT, sizeof(T) < sizeof(double) ? DGR_FP32_WAVES : 1) void k_fused(
+template <bool FACE, class C, bool HALO = false>
+__global__ __launch_bounds__(C::FT, DGR_FP32_WAVES) void k_fused(
     const StageIO io, const RhsParams prm, const DBlock *__restrict__ blocks,
     const dgr::AxisConsts *__restrict__ bconst, const Tile *__restrict__ tiles,
     const uint16_t *__restrict__ tabs, int dtab) {
-    // the region buffers sit at multiples of NREG doubles; with two buffers the
-    // FP32 kernel keeps FP64 data in the even-phase one only, the odd one FP32
-    constexpr bool DEEP = FusedCtx<FACE, C, T>::DEEP;
-    __shared__ double s_tile[DEEP ? 3 * C::NREG : C::NREG + (sizeof(T) < sizeof(double) ? (C::NREG + 1) / 2 : C::NREG)];
+    // the region buffers sit at multiples of NREG doubles; with two buffers
+    // FP64 data is kept in the even-phase one only, the odd one is FP32
+    constexpr bool DEEP = FusedCtx<FACE, C, float>::DEEP;
+    __shared__ double s_tile[DEEP ? 3 * C::NREG : C::NREG + (C::NREG + 1) / 2];
     __shared__ double s_dx[(DEEP ? 2 : 1) * C::NSDX];
     __shared__ double s_dy[(DEEP ? 2 : 1) * C::NSDY];
-    __shared__ T s_ko[NV * C::FT];
+    __shared__ float s_ko[NV * C::FT];
 
     const Tile tl = tiles[blockIdx.x];
     const DBlock B = blocks[tl.block];
-    fused_tile<FACE, C, T, HALO>(io, prm, tl, B, bconst + 3 * (size_t)tl.block, tabs, dtab, s_tile, s_dx, s_dy,
-                                 s_ko);
+    fused_tile<FACE, C, HALO>(io, prm, tl, B, bconst + 3 * (size_t)tl.block, tabs, dtab, s_tile, s_dx, s_dy, s_ko);
 }
 
 #ifndef DGR_F32_KERNELS
@@ -2135,14 +2118,14 @@ int fail(int code, const std::string &msg) {
 // scheduler, which was 3% faster on the one-wave FP64 kernels (the constraints'
 // are left of those) and spills the FP32 ones (measured).
 extern "C" __attribute__((visibility("hidden"))) void dgr_internal_fused_f32_kernels(const void **k) {
-    k[0] = reinterpret_cast<const void *>(&k_fused<false, CfgOf<float>::Wide, float>);
-    k[1] = reinterpret_cast<const void *>(&k_fused<false, CfgOf<float>::Thin, float>);
-    k[2] = reinterpret_cast<const void *>(&k_fused<false, CfgFull, float>);
-    k[3] = reinterpret_cast<const void *>(&k_fused<true, CfgOf<float>::Wide, float>);
-    k[4] = reinterpret_cast<const void *>(&k_fused<false, CfgOf<float>::Wide, float, true>);
-    k[5] = reinterpret_cast<const void *>(&k_fused<false, CfgOf<float>::Thin, float, true>);
-    k[6] = reinterpret_cast<const void *>(&k_fused<false, CfgFull, float, true>);
-    k[7] = reinterpret_cast<const void *>(&k_fused<true, CfgOf<float>::Wide, float, true>);
+    k[0] = reinterpret_cast<const void *>(&k_fused<false, F32Wide>);
+    k[1] = reinterpret_cast<const void *>(&k_fused<false, F32Thin>);
+    k[2] = reinterpret_cast<const void *>(&k_fused<false, CfgFull>);
+    k[3] = reinterpret_cast<const void *>(&k_fused<true, F32Wide>);
+    k[4] = reinterpret_cast<const void *>(&k_fused<false, F32Wide, true>);
+    k[5] = reinterpret_cast<const void *>(&k_fused<false, F32Thin, true>);
+    k[6] = reinterpret_cast<const void *>(&k_fused<false, CfgFull, true>);
+    k[7] = reinterpret_cast<const void *>(&k_fused<true, F32Wide, true>);
 }
 #elif defined(DGR_STREAM_KERNELS)
 // The FP64 stage kernels (stream_fp64.h), [halo][gauge][wide, full, face]
@@ -3027,32 +3010,6 @@ int run_chunks(dgr_plan *plan, const VarPtrs &state, const VarPtrs &rhs, const R
     return DGR_OK;
 }
 
-// Address of a fused kernel: the FP64 ones live in this unit, the FP32 ones
-// in the unit compiled with DGR_F32_KERNELS (see there).
-template <bool FACE, class C, typename T, bool HALO, bool GAUGE = false>
-const void *fused_kernel() {
-    if constexpr (sizeof(T) == sizeof(double)) {
-        static const void *const *tab = [] {
-            static const void *k[12];
-            dgr_internal_stream_kernels(k);
-            return k;
-        }();
-        return tab[6 * HALO + 3 * GAUGE + (FACE ? 2 : C::FT == CfgFull::FT ? 1 : 0)];
-    } else {
-        static_assert(!GAUGE, "the gauge variants are FP64 only");
-        static const void *const *tab = [] {
-            static const void *k[8];
-            dgr_internal_fused_f32_kernels(k);
-            return k;
-        }();
-        constexpr int h = HALO ? 4 : 0;  // the in-kernel refresh variants follow the others
-        if constexpr (FACE) return tab[h + 3];
-        else if constexpr (C::FT == CfgFull::FT) return tab[h + 2];
-        else if constexpr (C::FT == CfgThin::FT) return tab[h + 1];
-        else return tab[h];
-    }
-}
-
 StreamIO stream_io(const StageIO &io, const RhsParams &prm) {
     StreamIO r{};
     r.prm = prm;
@@ -3070,33 +3027,30 @@ StreamIO stream_io(const StageIO &io, const RhsParams &prm) {
     return r;
 }
 
-template <bool FACE, class C, typename T, bool HALO = false, bool GAUGE = false>
-void launch_fused(dgr_plan *plan, const Tile *tiles, const int *fg, int group, int dtab, const StageIO &io,
-                  const RhsParams &prm, hipStream_t st) {
+// A launch of k_stream on one group of tiles (kernel: its place among [wide, full, face]).
+template <bool HALO, bool GAUGE>
+void launch_kind(dgr_plan *plan, const Tile *tiles, const int *fg, int group, int kernel, const StreamIO &io,
+                 hipStream_t st) {
+    static const void *const *tab = [] {
+        static const void *k[12];
+        dgr_internal_stream_kernels(k);
+        return k;
+    }();
     const int n = fg[group + 1] - fg[group];
     if (!n) return;
-    // the kernel's parameters, in order (k_stream: without the RhsParams, which
-    // StreamIO holds, and the slot table)
-    constexpr bool FP64 = sizeof(T) == sizeof(double);
-    std::conditional_t<FP64, StreamIO, StageIO> a_io;
-    if constexpr (FP64) a_io = stream_io(io, prm);
-    else a_io = io;
-    RhsParams a_prm = prm;
-    const DBlock *a_blocks = plan->d_blocks;
-    const dgr::AxisConsts *a_bconst = plan->d_bconst;
+    StreamIO a_io = io;
     const Tile *a_tiles = tiles + fg[group];
-    const uint16_t *a_tabs = plan->d_tabs;
-    int a_dtab = dtab;
-    void *all[] = {&a_io, &a_prm, &a_blocks, &a_bconst, &a_tiles, &a_tabs, &a_dtab};
-    if (FP64) all[1] = all[0];
-    void **args = all + FP64;
-    // an FP64 launch on 6-7 deep tiles counts as the regular and the thin one it
-    // replaces, its time divided by their points; as the regular one only if the
-    // stage has no launch of regular tiles, so that each kind counts once a stage
-    const bool merged = FP64 && group == FG_FULL;
+    void *args[] = {&a_io, &plan->d_blocks, &plan->d_bconst, &a_tiles, &plan->d_tabs};
+    // a launch on 6-7 deep tiles counts as a regular and a thin one, its time
+    // divided by their points; as the regular one only if the stage has no launch
+    // of regular tiles, so that each kind counts once a stage
+    const bool merged = group == FG_FULL;
     timed(
         plan, 3 + (merged ? FG_WIDE : group), st,
-        [&] { (void)hipLaunchKernel(fused_kernel<FACE, C, T, HALO, GAUGE>(), dim3(n), dim3(C::FT), args, 0, st); },
+        [&] {
+            (void)hipLaunchKernel(tab[6 * HALO + 3 * GAUGE + kernel], dim3(n), dim3(merged ? SFull::FT : SWide::FT), args,
+                                  0, st);
+        },
         merged ? 3 + FG_THIN : -1, merged ? plan->full_regular : 1.0, !merged || fg[FG_WIDE + 1] == fg[FG_WIDE]);
 }
 
@@ -3129,6 +3083,7 @@ bool one_launch_tiled(const dgr_plan *plan, const std::array<int, 3> &n, int sch
 template <bool HALO, bool GAUGE>
 void launch_stream(dgr_plan *plan, const Tile *tiles, const int *fg, const StageIO &io, const RhsParams &prm,
                    hipStream_t st, bool one) {
+    const StreamIO sio = stream_io(io, prm);
     if (one) {
         const int nface = fg[FG_FULL] - fg[FG_FACE], nfull = fg[NFGROUP] - fg[FG_FULL], n = fg[NFGROUP] - fg[FG_WIDE];
         static const void *const *tab = [] {
@@ -3136,38 +3091,52 @@ void launch_stream(dgr_plan *plan, const Tile *tiles, const int *fg, const Stage
             dgr_internal_small_kernels(k);
             return k;
         }();
-        StreamIO a_io = stream_io(io, prm);
+        StreamIO a_io = sio;
         const Tile *a_tiles = tiles + fg[FG_WIDE];
         int face0 = n - nface - nfull, full0 = n - nfull;
         void *args[] = {&a_io, &plan->d_blocks, &plan->d_bconst, &a_tiles, &plan->d_tabs, &face0, &full0};
         (void)hipLaunchKernel(tab[2 * HALO + GAUGE], dim3(n), dim3(SFull::FT), args, 0, st);
         return;
     }
-    launch_fused<false, CfgWide, double, HALO, GAUGE>(plan, tiles, fg, FG_WIDE, plan->dtab_wide, io, prm, st);
-    launch_fused<false, CfgFull, double, HALO, GAUGE>(plan, tiles, fg, FG_FULL, plan->dtab_full, io, prm, st);
-    launch_fused<true, CfgWide, double, HALO, GAUGE>(plan, tiles, fg, FG_FACE, plan->dtab_wide, io, prm, st);
+    launch_kind<HALO, GAUGE>(plan, tiles, fg, FG_WIDE, 0, sio, st);
+    launch_kind<HALO, GAUGE>(plan, tiles, fg, FG_FULL, 1, sio, st);
+    launch_kind<HALO, GAUGE>(plan, tiles, fg, FG_FACE, 2, sio, st);
 }
 
-template <typename T>
-void launch_fused_all(dgr_plan *plan, const Tile *tiles, const int *fg, const StageIO &io, const RhsParams &prm,
-                      hipStream_t st, bool one = false) {
-    if constexpr (sizeof(T) == sizeof(double)) {
-        const bool gauge = gauge_variant(prm);  // the reference's other builds (FP64 only)
-        if (io.nbo && gauge) launch_stream<true, true>(plan, tiles, fg, io, prm, st, one);
-        else if (io.nbo) launch_stream<true, false>(plan, tiles, fg, io, prm, st, one);
-        else if (gauge) launch_stream<false, true>(plan, tiles, fg, io, prm, st, one);
-        else launch_stream<false, false>(plan, tiles, fg, io, prm, st, one);
-    } else if (io.nbo) {  // the padding refresh inside the stage kernel
-        launch_fused<false, CfgOf<float>::Wide, T, true>(plan, tiles, fg, FG_WIDE, plan->dtab_wide, io, prm, st);
-        launch_fused<false, CfgOf<float>::Thin, T, true>(plan, tiles, fg, FG_THIN, plan->dtab_thin, io, prm, st);
-        launch_fused<false, CfgFull, T, true>(plan, tiles, fg, FG_FULL, plan->dtab_full, io, prm, st);
-        launch_fused<true, CfgOf<float>::Wide, T, true>(plan, tiles, fg, FG_FACE, plan->dtab_wide, io, prm, st);
-    } else {
-        launch_fused<false, CfgOf<float>::Wide, T>(plan, tiles, fg, FG_WIDE, plan->dtab_wide, io, prm, st);
-        launch_fused<false, CfgOf<float>::Thin, T>(plan, tiles, fg, FG_THIN, plan->dtab_thin, io, prm, st);
-        launch_fused<false, CfgFull, T>(plan, tiles, fg, FG_FULL, plan->dtab_full, io, prm, st);
-        launch_fused<true, CfgOf<float>::Wide, T>(plan, tiles, fg, FG_FACE, plan->dtab_wide, io, prm, st);
-    }
+// The launches of one FP64 tile list.
+void launch_fp64(dgr_plan *plan, const Tile *tiles, const int *fg, const StageIO &io, const RhsParams &prm,
+                 hipStream_t st, bool one) {
+    const bool gauge = gauge_variant(prm);  // the reference's other builds (FP64 only)
+    if (io.nbo && gauge) launch_stream<true, true>(plan, tiles, fg, io, prm, st, one);
+    else if (io.nbo) launch_stream<true, false>(plan, tiles, fg, io, prm, st, one);
+    else if (gauge) launch_stream<false, true>(plan, tiles, fg, io, prm, st, one);
+    else launch_stream<false, false>(plan, tiles, fg, io, prm, st, one);
+}
+
+// The launches of one mixed-precision tile list (k_fused: the unit compiled with
+// DGR_F32_KERNELS holds the kernels, the in-kernel refresh ones from 4 on).
+void launch_mixed(dgr_plan *plan, const Tile *tiles, const int *fg, const StageIO &io, const RhsParams &prm,
+                  hipStream_t st) {
+    static const void *const *tab = [] {
+        static const void *k[8];
+        dgr_internal_fused_f32_kernels(k);
+        return k;
+    }();
+    auto launch = [&](int group, int kernel, int threads, int dtab) {
+        const int n = fg[group + 1] - fg[group];
+        if (!n) return;
+        StageIO a_io = io;
+        RhsParams a_prm = prm;
+        const Tile *a_tiles = tiles + fg[group];
+        void *args[] = {&a_io, &a_prm, &plan->d_blocks, &plan->d_bconst, &a_tiles, &plan->d_tabs, &dtab};
+        timed(plan, 3 + group, st, [&] {
+            (void)hipLaunchKernel(tab[kernel + (io.nbo ? 4 : 0)], dim3(n), dim3(threads), args, 0, st);
+        });
+    };
+    launch(FG_WIDE, 0, F32Wide::FT, plan->dtab_wide);
+    launch(FG_THIN, 1, F32Thin::FT, plan->dtab_thin);
+    launch(FG_FULL, 2, CfgFull::FT, plan->dtab_full);
+    launch(FG_FACE, 3, F32Wide::FT, plan->dtab_wide);
 }
 
 int run_fused(dgr_plan *plan, const StageIO &io, const RhsParams &prm, hipStream_t st) {
@@ -3175,11 +3144,10 @@ int run_fused(dgr_plan *plan, const StageIO &io, const RhsParams &prm, hipStream
         return fail(DGR_E_INVALID, "the eta function, the Rochester gauge and the slow-start lapse "
                                    "(eta_func, rochester, ssl) need FP64 precision");
     if (plan->precision == DGR_PRECISION_MIXED)
-        launch_fused_all<float>(plan, plan->d_ftiles[1], plan->fgroup[1], io, prm, st);
+        launch_mixed(plan, plan->d_ftiles[1], plan->fgroup[1], io, prm, st);
     else
         // (with timing on a launch a kind, so that each has its own time)
-        launch_fused_all<double>(plan, plan->d_ftiles[0], plan->fgroup[0], io, prm, st,
-                                 one_launch(plan->fgroup[0]) && !plan->timing);
+        launch_fp64(plan, plan->d_ftiles[0], plan->fgroup[0], io, prm, st, one_launch(plan->fgroup[0]) && !plan->timing);
     HIP_OK(hipGetLastError());
     return DGR_OK;
 }
@@ -3263,8 +3231,8 @@ int dgr_plan_autotune(dgr_plan *plan, double *const *d_rhs, const double *const 
                 float ms = 0.f;
                 for (int rep = 0; rep < 4; rep++) {  // a warm-up, then the best of three
                     HIP_OK(hipEventRecord(e0, st));
-                    if (p) launch_fused_all<float>(plan, d_t, fg, io, prm, st);
-                    else launch_fused_all<double>(plan, d_t, fg, io, prm, st, one);
+                    if (p) launch_mixed(plan, d_t, fg, io, prm, st);
+                    else launch_fp64(plan, d_t, fg, io, prm, st, one);
                     HIP_OK(hipGetLastError());
                     HIP_OK(hipEventRecord(e1, st));
                     HIP_OK(hipEventSynchronize(e1));
