@@ -187,8 +187,12 @@ int dgr_plan_move_block(dgr_plan *plan, uint32_t b, uint64_t offset, const doubl
  * tiles of blocks without flagged faces, 4 on thin tiles, 5 on tiles of
  * blocks with flagged faces, 6 the mixed-precision kernel on 7 x 7 x 7 tiles
  * of blocks without flagged faces (it replaces 3 and 4 in that precision).
- * An FP64 launch on tiles of a regular part with its 1-2 point remainder counts
- * in 3 and in 4, its time divided by the points of the two. */
+ * In FP64 a remainder of 1-2 points has no launch of its own: it is part of a
+ * launch on 6-7 deep tiles. That launch's time is entered under 3 and 4, divided
+ * by the points of its first 5 planes and of the rest, and 3 and 4 count one
+ * launch a stage each where the stage has such tiles (so 3 holds the sum of two
+ * launches where it has regular tiles as well). The sum of 3 and 4 is the time
+ * the device took on blocks without flagged faces; neither alone is. */
 #define DGR_TIMING_KINDS 7
 int dgr_plan_set_timing(dgr_plan *plan, int enable);
 int dgr_plan_kernel_times(dgr_plan *plan, double *ms, int64_t *launches);
