@@ -21,9 +21,9 @@ Beside it, in the same line:
                 without flagged faces; in FP64 one launch a stage, or two where
                 there are 7x7x5 and 7x7x7 tiles, taken together) against HBM:
                 algorithmic bytes per stage (per block 192 n^3 for reading the
-                padded state once, per interior point 192 for the RHS and 768 for
-                the RK stage update, split over the kinds by the points each
-                covers) over its average time a stage, measured with HIP
+                padded state once, per interior point 624 for the RK stage
+                update, the mean of the four stages, split over the kinds by the
+                points each covers) over its average time a stage, measured with HIP
                 events on the launch stream; `traffic` is the HBM bytes of the
                 same launches measured with rocprofv3 counters (profiles/), when
                 a summary measured on the current kernel sources is committed

@@ -270,13 +270,15 @@ def puncture_octree(scale: float = 0.42, align: int = 1) -> np.ndarray:
 
 
 def stage_bytes(t: np.ndarray) -> float:
-    """Algorithmic HBM bytes of one fused RK stage over all blocks: each padded
-    FP64 state read once (192 n^3 per block), per interior point the RHS
-    produced once (192) and the stage update (read u0, read and write the
-    accumulator, write the next stage: 768)."""
+    """HBM bytes that one RK stage moves at least, the mean of a step's four, over all
+    blocks: each padded FP64 state read once (192 n^3 per block) and, per
+    interior point, the stage update: stage 0 writes the step's start, the
+    accumulator and the next stage (576), stages 1 and 2 read the first two and
+    write the last two (768), stage 3 reads the accumulator and writes the result
+    (384). The right-hand side itself is never written."""
     n3 = np.prod(t["sz"].astype(np.float64), axis=1)
     m3 = np.prod(t["sz"].astype(np.float64) - 2 * PW, axis=1)
-    return float((192.0 * n3 + 960.0 * m3).sum())
+    return float((192.0 * n3 + 624.0 * m3).sum())
 
 
 def fused_kind_bytes(t: np.ndarray, precision: str = "fp64") -> dict:

@@ -48,3 +48,14 @@ def test_mixed_launches_are_entries_as_they_ran():
     r = line(t, {"fused_full": (8 * 0.9, 8), "fused_face": (0.0, 0)}, 8, "mixed")
     assert r["launch_ms"] == pytest.approx(0.9)
     assert r["algorithmic_bytes_per_launch"] == pytest.approx(W.stage_bytes(t))
+
+
+def test_stage_bytes_are_what_four_stages_move():
+    """Per interior point: stage 0 writes the step's start, the accumulator and the
+    next stage (3 x 192), stages 1 and 2 read the first two and write the last two
+    (4 x 192), stage 3 reads the accumulator and writes the result (2 x 192); each
+    reads its padded state once. No stage writes a right-hand side."""
+    t = blocks([(13, 13, 13), (19, 14, 31)])
+    padded = 13 ** 3 + 19 * 14 * 31
+    inner = 7 ** 3 + 13 * 8 * 25
+    assert 4 * W.stage_bytes(t) == 192 * (4 * padded + (3 + 4 + 4 + 2) * inner)
