@@ -422,7 +422,7 @@ def halo_rate(wl, plan, state, stream, calls=20):
     ms = e0.elapsed_time(e1) / calls
     return {"links": int((nbr >= 0).sum()), "padding_points_filled": pts, "bytes_per_launch": byts,
             "ms_per_launch": round(ms, 4), "achieved_GBs": round(byts / ms / 1e6, 1),
-            "use": ("FP64 RK4 stages read linked padding inside k_fused (HALO variant); this fill "
+            "use": ("RK4 stages read linked padding inside the stage kernels (HALO variants); this fill "
                     "runs once per RK4 call, leaving the caller's padding refreshed")}
 
 
@@ -455,7 +455,7 @@ def fill_rate(wl, plan, state, stream, calls=10):
     pts = linked + ncopy + ninterp
     return {"linked_points": linked, "copied_points": ncopy, "interpolated_points": ninterp,
             "ms_per_call": round(ms, 4), "copy_equivalent_GBs": round(pts * 24 * 16 / ms / 1e6, 1),
-            "use": ("RK4 stages read same-level padding inside k_fused (HALO variant) and get the rest "
+            "use": ("RK4 stages read same-level padding inside the stage kernels (HALO variants) and get the rest "
                     "written before each stage by k_fill_copy and k_fill_interp; this full fill runs once per RK4 call")}
 
 

@@ -555,21 +555,22 @@ __global__ __launch_bounds__(NTHREADS) void k_face(VarPtrs u, VarPtrs rhs, RKArg
 }
 
 // -------------------------------------------------------------------------
-// k_fused: derivatives, equations, KO, BC and the stage update in one kernel.
-// One workgroup per tile of at most 7 x 7 x 5 points, one point per thread
-// (threads beyond the tile's points shadow its last point and store nothing).
-// The 24 variables stream through LDS in the phase order of
-// bssn_rhs_phased.h: while phase K works on variable V (staged in LDS buffer
-// K&1), the next variable's region is already in flight into registers.
-// Every thread's own field values sit in LDS for the equations, its KO term
-// (on flagged faces: boundary value plus KO term) is left in LDS, and the
-// right-hand side is combined with both in one batched epilogue.
+// k_fused (FP32): derivatives, equations, KO, BC and the stage update in one
+// kernel; k_cons_fused (FP64): the constraints on the same machinery.
+// One workgroup per tile of at most 7 x 7 x 7 points, one point per thread
+// (threads beyond the tile's points shadow one of them and store nothing).
+// The variables stream through LDS in the phase order of bssn_rhs_phased.h
+// or bssn_cons_phased.h: while phase K works on variable V, staged in LDS, the
+// next variable's region is already in flight into registers. A thread keeps
+// its own field values in registers; k_fused leaves its KO term (on flagged
+// faces: boundary value plus KO term) in LDS and combines the right-hand side
+// with it in one batched epilogue.
 //
-// Instruction economy matters more than usual here: the equations need about
-// 430 registers per lane, so a SIMD runs a single wave and every instruction
-// costs a full issue slot. LDS strides are compile-time (region 13 x 13 x
-// (ez+6)), stencil constants come precomputed per block, and face closures
-// sit behind a branch that is uniform over the tile.
+// Registers bound both: the FP32 equations fill 256 (two waves a SIMD, with
+// spills), the FP64 constraints more (one wave), so instructions are few. LDS
+// strides are compile-time (region 13 x 13 x (ez+6)), stencil constants come
+// precomputed per block, and face closures sit behind a branch that is uniform
+// over the tile.
 // -------------------------------------------------------------------------
 constexpr int FRX = RMAX, FRXY = RMAX * RMAX;  // LDS strides of the staged region (13, 169)
 // D_x u (tile x, region y, region z) and D_y u (tile x, tile y, region z) use
@@ -628,14 +629,16 @@ static_assert(sizeof(double) * (3 * CfgFull::NREG + 2 * (CfgFull::NSDX + CfgFull
 static_assert(7 * 7 * CfgWide::FZ <= CfgWide::FT && 7 * 7 * CfgThin::FZ <= CfgThin::FT &&
                   7 * 7 * CfgFull::FZ <= CfgFull::FT,
               "one point per thread");
-// tile groups of the fused path, one launch each (FULL: FP32 only)
+// tile groups of the fused path, one launch each. THIN: mixed precision only;
+// FULL: in FP64 the 6-7 deep tiles of SCH_WT, in mixed precision SCH_FULL's
 enum { FG_WIDE = 0, FG_THIN = 1, FG_FACE = 2, FG_FULL = 3, NFGROUP = 4 };
 // Tilings of a block without flagged faces, chosen per block size and
 // precision (dgr_plan_autotune measures them). x and y are always cut into
 // near-equal parts of at most 7 points; along z:
-//   SCH_WT   parts of 5, a remainder of 1-2 points in thin tiles (128 threads)
+//   SCH_WT   parts of 5, a remainder of 1-2 points in thin tiles (128 threads;
+//            mixed precision) or in a 6-7 deep tile with the 5 before it (FP64)
 //   SCH_W    near-equal parts of at most 5, all regular tiles
-//   SCH_FULL near-equal parts of at most 7 (384 threads; FP32 only)
+//   SCH_FULL near-equal parts of at most 7 (384 threads; mixed precision only)
 enum { SCH_WT = 0, SCH_W = 1, SCH_FULL = 2, NSCHEME = 3 };
 
 // Where a stage reads its state and writes its results. Stage buffers hold
@@ -662,8 +665,8 @@ struct StageIO {
     int enforce_stage;
     int *err;
     // 27 per block: the offset of the same-level neighbour in each direction
-    // (-1 for none), read only by the HALO instantiation of k_fused, which
-    // stages region points inside a linked neighbour from that neighbour's
+    // (-1 for none), read only by the HALO instantiations, which
+    // stage region points inside a linked neighbour from that neighbour's
     // interior instead of the block's own padding
     const int64_t *nbo;
 };
@@ -719,7 +722,7 @@ struct FusedCtx {
     // LDS source offsets of this thread's D_x / D_y evaluations
     int dxw[DXIT], dyw[DYIT];  // where this thread's D_x / D_y evaluations go (see dtable)
     T d1v[3], d2v[6];
-    // FP64: the interior stencil constants of the block (1/(60h), 1/(180h^2),
+    // FP64 (the constraints): the interior stencil constants of the block (1/(60h), 1/(180h^2),
     // KO prefactor per axis) held in vector registers. Left to the compiler
     // they are scalar loads re-issued near every use, and since scalar and LDS
     // loads share one wait counter, each re-issue drains the LDS queue (+1.2%
@@ -782,8 +785,8 @@ struct FusedCtx {
     template <int V>
     using Stage = std::conditional_t<(sizeof(T) < sizeof(double) && (V == 0 || V == 1)), double, T>;
 
-    // One barrier per phase where LDS allows it (DEEP: the FP64 256-thread and
-    // FP32 384-thread kernels, which hold one workgroup per CU anyway): three
+    // One barrier per phase where LDS allows it (DEEP: the 256-thread constraint
+    // and 384-thread FP32 kernels, which hold one workgroup per CU anyway): three
     // region buffers and two D_x / D_y buffers, so phase K stages variable K+1
     // before its single barrier, and phase K+1's D_x / D_y and region stencils
     // follow phase K's equations with no barrier between them (the scheduler
@@ -2201,7 +2204,7 @@ struct dgr_plan {
     double *d_W = nullptr;
     int64_t max_chunk_points = 0;
     double *d_stage = nullptr;  // split path RK4: 2 * 24 * szpdof (stage state, accumulator)
-    bool fused = true;          // k_fused (default) or the split k_derivs/k_rhs path (DGR_KERNEL=split)
+    bool fused = true;          // a stage in one kernel (default) or the split k_derivs/k_rhs path (DGR_KERNEL=split)
     int precision = DGR_PRECISION_FP64;  // arithmetic of the fused kernel
     // tile lists per precision (0 FP64, 1 mixed), XCD-grouped, group k in
     // [fgroup[p][k], fgroup[p][k+1]), each interior block tiled by the scheme
@@ -2212,12 +2215,12 @@ struct dgr_plan {
     std::vector<DBlock> hblocks;                  // host copy of the block table
     std::map<std::array<int, 4>, int> lane_off;   // lane table offset per (ex, ey, ez, threads)
     std::map<std::array<int, 3>, int> stage_off;  // staging table offset per (ex, threads, halo)
-    dgr::AxisConsts *d_bconst = nullptr;  // k_fused: x, y, z stencil constants per block
-    uint16_t *d_tabs = nullptr;           // k_fused: lane tables per tile shape, slot tables per config
+    dgr::AxisConsts *d_bconst = nullptr;  // fused path: x, y, z stencil constants per block
+    uint16_t *d_tabs = nullptr;           // fused path: lane, staging and slot tables
     int dtab_wide = 0, dtab_thin = 0, dtab_full = 0;  // offsets of the configurations' slot tables
     std::vector<int> hnbr;      // same-level neighbour table, 27 per block (built on first use)
     int *d_nbr = nullptr;       // its device copy
-    int64_t *d_nbo = nullptr;   // the same as neighbour block offsets (-1 for none), for k_fused
+    int64_t *d_nbo = nullptr;   // the same as neighbour block offsets (-1 for none), for the HALO kernels
     int64_t nlinks = -1;        // links in the table (-1: not built yet)
     int2 *d_halo_wg = nullptr;  // k_halo_fill's workgroups: (block, chunk) of the linked blocks
     int64_t nhalo_wg = 0;
@@ -2228,12 +2231,12 @@ struct dgr_plan {
     int64_t nfill_interp = 0;   // of which interpolations (they follow the copies)
     FillGroup *d_fill_groups = nullptr;  // the interpolations grouped by coarse element
     int64_t nfill_groups = 0;
-    double *d_istage = nullptr; // k_fused RK4: 2 * 24 * interior (u0 copy, accumulator)
+    double *d_istage = nullptr; // fused RK4: 2 * 24 * interior (u0 copy, accumulator)
     double *d_rk45 = nullptr;   // dgr_rk45_step: the six stages' right-hand sides, 6 * 24 * interior
     unsigned long long *d_rk45_emax = nullptr;  // dgr_rk45_step: the error estimate's bits
     double *d_ssl = nullptr;    // dgr_rk4_steps with the slow-start lapse: {time, exp(-time^2/800)}
     unsigned long long *d_range = nullptr;      // dgr_variable_range: min key, max key, non-finite count
-    double *d_wstate = nullptr; // k_fused RK4: 24 * szpdof, the padded work state W
+    double *d_wstate = nullptr; // fused RK4: 24 * szpdof, the padded work state W
     int *d_err = nullptr;
     // dgr_rk4_steps: one RK4 step captured as a graph, valid for the arguments in rk4_key
     hipStream_t cap_stream = nullptr;
@@ -2442,9 +2445,10 @@ struct TileGroup {
 // the 7-deep shape: a thin tile of its own stages and differentiates 6 planes
 // of halo for its 2 (on 13^3 blocks, 4096 of them, the two launches of a stage
 // fetched 3.3 GB where one fetches 2.4). Blocks
-// with flagged faces are cut along z into near-equal parts of at most 5 (each
-// >= 4 points, so the one-sided closures, which reach 5 points along their
-// axis, stay inside the staged region), whatever the scheme.
+// with flagged faces are cut along z into near-equal parts of at most 5, whatever
+// the scheme (7 as 4 + 3, 11 as 4 + 4 + 3): at least 3 points, so
+// the one-sided closures, for the 3 points next to a face from the 6 values next
+// to it, stay inside the one tile that meets the face and its staged 3-point halo.
 void block_tiles(const DBlock &d, uint32_t b, int p, int sch, TileGroup *per, size_t slot) {
     std::vector<std::pair<int, int>> px, py, pz;
     split_axis_max(d.n[0] - 6, TMAX, px);
@@ -2722,7 +2726,7 @@ int dgr_plan_create(int device, const dgr_block *blocks, uint32_t nblocks, uint6
     close_chunk();
     plan->nwg_total = (int)wg_tile.size();
 
-    // k_fused: slot tables per configuration, lane tables for every tile
+    // fused path: slot tables per configuration, lane and staging tables for every tile
     // shape any tiling can produce (one block per size and kind suffices);
     // the tile lists themselves are built per precision after the uploads
     plan->hblocks = hb;
@@ -3716,7 +3720,7 @@ int launch_padding_refresh(dgr_plan *plan, const VarPtrs &u, hipStream_t st) {
 constexpr uint64_t HALO_POINTS_MAX = (1ull << 29) - 16;
 
 // With the padding refresh on, stages read linked padding straight from the
-// neighbours (k_fused<..., HALO>); plans whose variables hold 2^29 points or
+// neighbours (the HALO kernels); plans whose variables hold 2^29 points or
 // more get the padding copied in by k_halo_fill before each stage instead.
 bool halo_in_kernel(const dgr_plan *plan) {
     // the HALO kernels address the whole variable with 32-bit byte offsets;

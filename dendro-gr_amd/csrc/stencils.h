@@ -5,7 +5,10 @@
 // domain boundary. Each expression keeps the term order of the reference
 // stencil it restates, and floating-point contraction is off, so the sums
 // round exactly as the reference's do (the right-hand sides of near-puncture
-// data are small differences of these sums, so FMA rounding would show).
+// data are small differences of these sums, so FMA rounding would show). One
+// exception: ko_face multiplies its sums by reciprocals of the boundary
+// divisors where the reference, and ko_edge, divide by them, which may differ
+// in the last bit.
 #pragma once
 
 namespace dgr {
@@ -259,6 +262,9 @@ __device__ __forceinline__ double d2_face(const double *e, double r, int l, doub
                         : (-e[0] + 16.0 * e[1] - 30.0 * e[2] + 16.0 * e[3] - e[4]) * by12;
     return l == 0 ? a : l == 1 ? b : l == 2 ? c : r;
 }
+// (by reciprocals, for a division is ~30 instructions in FP64: the right-hand side
+// of 200 ragged blocks, 30% of them flagged, is 2.3e-13 from
+// values computed apart with either, that of one 19^3 block 1.9e-13)
 template <typename K>
 __device__ __forceinline__ double ko_face(const double *e, double r, int l, const K &k) {
 #pragma clang fp contract(off)

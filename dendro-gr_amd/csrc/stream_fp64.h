@@ -20,9 +20,9 @@
 // address units were 84% busy while the vector units idled at 28%. So a
 // region is read 16 bytes a lane, the corners no stencil reaches are left out,
 // and the interior buffers lie in lane order (stage_table, StreamIO).
-// Measured, a whole RK4 step, against the one-wave kernel this replaces (126
-// live doubles, 480 registers): 30.0 M points of uneven octree 94.3 -> 65.2 ms;
-// 4096 blocks of 13^3 5.05 -> 3.79 ms (its stage alone 1.06 -> 0.75); the
+// Measured, a whole RK4 step with its padding copy, against the one-wave kernel
+// this replaces (126 live doubles, 480 registers): 30.0 M points of uneven octree
+// 95.6 -> 60.9 ms; 4096 blocks of 13^3 5.05 -> 3.57 ms (its stage alone 1.06 -> 0.78); the
 // right-hand side of 200 ragged blocks, a third on the boundary, 1.88 -> 0.99 ms;
 // one 19^3 block with every face flagged 118 -> 83 us (1.12 ms and 115 us before
 // D_x and D_y went along lines, SCfg::XLINES).
