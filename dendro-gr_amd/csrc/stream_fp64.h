@@ -20,9 +20,14 @@
 // address units were 84% busy while the vector units idled at 28%. So a
 // region is read 16 bytes a lane, the corners no stencil reaches are left out,
 // and the interior buffers lie in lane order (stage_table, StreamIO).
+// Busy now, of a launch's cycles: 7x7x5 tiles (octree) the texture address units 76%,
+// LDS 41%, the vector units 40%; 7x7x7 tiles 43-54%, 26-29% and 28-32%, their six waves
+// on four SIMDs waiting 45% of their time (LDS, memory, the barrier); flagged tiles 24%,
+// 22% and 31% on 288 KB of code, of which 3-4% of the fetches miss the 64 KB
+// instruction cache (the others' 62 KB fit: 0.1%).
 // Measured, a whole RK4 step with its padding copy, against the one-wave kernel
 // this replaces (126 live doubles, 480 registers): 30.0 M points of uneven octree
-// 95.6 -> 60.9 ms; 4096 blocks of 13^3 5.05 -> 3.57 ms (its stage alone 1.06 -> 0.78); the
+// 95.6 -> 60.9 ms; 4096 blocks of 13^3 5.05 -> 3.57 ms (its stage alone 1.06 -> 0.77); the
 // right-hand side of 200 ragged blocks, a third on the boundary, 1.88 -> 0.99 ms;
 // one 19^3 block with every face flagged 118 -> 83 us (1.12 ms and 115 us before
 // D_x and D_y went along lines, SCfg::XLINES).
