@@ -263,7 +263,7 @@ __device__ __forceinline__ double d2_face(const double *e, double r, int l, doub
     return l == 0 ? a : l == 1 ? b : l == 2 ? c : r;
 }
 // (by reciprocals, for a division is ~30 instructions in FP64: the right-hand side
-// of 200 ragged blocks, 30% of them flagged, is 2.3e-13 from
+// of 200 ragged blocks, 28% of them flagged, is 2.3e-13 from
 // values computed apart with either, that of one 19^3 block 1.9e-13)
 template <typename K>
 __device__ __forceinline__ double ko_face(const double *e, double r, int l, const K &k) {

@@ -28,7 +28,7 @@
 // Measured, a whole RK4 step with its padding copy, against the one-wave kernel
 // this replaces (126 live doubles, 480 registers): 30.0 M points of uneven octree
 // 95.6 -> 60.9 ms; 4096 blocks of 13^3 5.05 -> 3.57 ms (its stage alone 1.06 -> 0.77); the
-// right-hand side of 200 ragged blocks, a third on the boundary, 1.88 -> 0.99 ms;
+// right-hand side of 200 ragged blocks, 28% of them flagged, 1.88 -> 0.99 ms;
 // one 19^3 block with every face flagged 118 -> 83 us (1.12 ms and 115 us before
 // D_x and D_y went along lines, SCfg::XLINES).
 
