@@ -295,7 +295,7 @@ class Plan:
 
     def set_precision(self, precision: str):
         """'fp64' (default) or 'mixed' (FP32 derivatives/equations, FP64 state;
-        less exact, and 0.77-0.81 of the FP64 rate)."""
+        less exact, and 0.77-0.86 of the FP64 rate)."""
         _check(load().dgr_plan_set_precision(self._h, PRECISION[precision]), "dgr_plan_set_precision")
 
     def autotune(self, out, state, params: BssnParams, stream=None):

@@ -122,7 +122,7 @@ int dgr_plan_destroy(dgr_plan *plan);
  * (the value at the tile region's first point), while the state, the RK stage
  * accumulation and the constraint enforcement stay FP64; the right-hand side
  * is widened to FP64 before it is stored or used. Fused path only. It is the less
- * exact and also the slower of the two: 0.77-0.81 of the FP64 rate of RK4 steps,
+ * exact and also the slower of the two: 0.77-0.86 of the FP64 rate of RK4 steps,
  * on 1.4 to 120 M points, uniform or octree, padding frozen or refreshed. */
 #define DGR_PRECISION_FP64 0
 #define DGR_PRECISION_MIXED 1
